@@ -22,6 +22,7 @@ struct GemvParams {
   uint32_t x_bytes, w_bytes;
   int M, N, K, KB;                 // KB = ceil(K / 64)
   int split;                       // waves per group of n-tiles, each taking every split-th k-block
+  int units, gpb;                  // one row: units of weight rows, and those of one workgroup
   // Activation epilogue (ACT template argument): 1, GELU pair: the weight is [gate; up] stacked
   // (N = 2I, I a multiple of 16) and y [M, I] = bf16(bf16(gelu_tanh(g)) * u) with g, u the bf16
   // outputs of the gate and up rows; 2, GELU times a multiplier: y = bf16(bf16(gelu_tanh(g)) * mul)
@@ -35,7 +36,7 @@ struct GemvParams {
   // (no res: h = bf16(rms(pro_y) * w1)).  Workgroup 0 stores h when pro_h is set.
   const uint16_t* pro_y; const uint16_t* pro_res; const uint16_t* pro_w1; const uint16_t* pro_scalar;
   const uint16_t* pro_w2; uint16_t* pro_h;
-  float pro_eps; int pro_norm2, pro_ch;  // pro_ch: the row kernel's 8-element chunks per lane for K
+  float pro_eps; int pro_norm2;
   // Attention-merge prologue (PRO == 4, M = 1): the activation row is one token's decode attention
   // output [H * D], merged from the split-key kernel's chunk partials (part_o [KV][nchunk_grid][G][D],
   // part_ml [KV][nchunk_grid][G][2]) as attn_decode_merge_kernel merges them, for at most
@@ -44,18 +45,21 @@ struct GemvParams {
   int m_window, m_nchunk_grid, m_G, m_D, m_chunk; float m_c;
 };
 
+// The longest activation row that the one-row kernels hold in LDS (24 KiB).
+constexpr int GEMV_ROW_MAX = 12288;
+// Heads that the merge prologue makes chunk weights for: H * D <= 4096 at head_dim 128.
+constexpr int MERGE_HEADS = 32;
+
 // The merge prologue.  For at most 16 chunks attn_decode_merge_kernel's sums reduce to fixed orders,
 // taken here: per head, its chunk weights w_c = exp2(M_c c - M c) and the weighted l over a 16-leaf
 // tree (t + 8, t + 4, t + 2, t + 1), made once per workgroup by one thread per head into mw
-// [16 heads][17] (w_0 .. w_15, then 1 / l); per element, the chunks in order, each term
+// [MERGE_HEADS][17] (w_0 .. w_15, then 1 / l); per element, the chunks in order, each term
 // fma(w_c, o_c, 0), a +0 after them when fewer than 16 are live (the merge kernel's empty parts).
 // Each thread makes elements e, e + 1 of the row (one head, columns d, d + 1); the partials of its
 // first pair are fetched before the weights are made.
 __device__ __forceinline__ void gemv_attn_merge_row(const GemvParams& p, uint16_t* xs, float* mw) {
   constexpr int NC = DEC_MERGE_IN_GEMV_CHUNKS;
   const int pos = *p.m_pos;
-  const int klo = p.m_window > 0 ? max(0, pos - p.m_window + 1) : 0;
-  const int nchunk = max(0, min((pos - klo) / p.m_chunk + 1, p.m_nchunk_grid));
   const int H = p.K / p.m_D;
   auto head_base = [&](int h) { return int64_t(h / p.m_G) * p.m_nchunk_grid * p.m_G + h % p.m_G; };
   // this thread's first pair: its partials now
@@ -66,20 +70,30 @@ __device__ __forceinline__ void gemv_attn_merge_row(const GemvParams& p, uint16_
     const int64_t hb = head_base(h);
 #pragma unroll
     for (int c = 0; c < NC; ++c)
-      oc[c] = (c < nchunk && e < p.K) ? *reinterpret_cast<const v2f*>(p.m_po + (hb + int64_t(c) * p.m_G) * p.m_D + d)
-                                      : v2f{0.0f, 0.0f};
+      oc[c] = (c < p.m_nchunk_grid && e < p.K)
+                  ? *reinterpret_cast<const v2f*>(p.m_po + (hb + int64_t(c) * p.m_G) * p.m_D + d)
+                  : v2f{0.0f, 0.0f};
   };
+  // The loads cover every chunk the grid has, so none waits for the position; chunks that are not
+  // live yet (their partials hold old values) are left out afterwards.
   fetch(e);
+  v2f ml[NC];
+  const int hw = min(int(threadIdx.x), H - 1);
+  if (int(threadIdx.x) < H) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+      ml[c] = c < p.m_nchunk_grid ? *reinterpret_cast<const v2f*>(p.m_ml + (head_base(hw) + int64_t(c) * p.m_G) * 2)
+                                  : v2f{0.0f, 0.0f};
+  }
+  const int klo = p.m_window > 0 ? max(0, pos - p.m_window + 1) : 0;
+  const int nchunk = max(0, min((pos - klo) / p.m_chunk + 1, p.m_nchunk_grid));
   if (int(threadIdx.x) < H) {
     const int h = int(threadIdx.x);
-    const int64_t hb = head_base(h);
     float mc[NC], lc[NC];
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-      const v2f ml = c < nchunk ? *reinterpret_cast<const v2f*>(p.m_ml + (hb + int64_t(c) * p.m_G) * 2)
-                                : v2f{-__builtin_inff(), 0.0f};
-      mc[c] = ml[0];
-      lc[c] = ml[1];
+      mc[c] = c < nchunk ? ml[c][0] : -__builtin_inff();
+      lc[c] = c < nchunk ? ml[c][1] : 0.0f;
     }
     float M = -__builtin_inff();
 #pragma unroll
@@ -122,98 +136,99 @@ __device__ __forceinline__ void gemv_attn_merge_row(const GemvParams& p, uint16_
   }
 }
 
-// The row prologue on one wave, in the arithmetic and order of the row kernel's one-wave rows
-// (row_chain_kernel with 64 threads, rowops.hip): lane t holds chunks c < CH of 8 elements at
-// k = 8 * (64 c + t); the sums of squares are added chunk by chunk, element by element, then across
-// the wave by wave_sum_dpp.  Its operands are fetched first (RowIn::load), before the kernel issues
-// its weight loads, so the arithmetic (RowIn::make) waits for them alone; the result goes to
-// xs [CH * 512] bf16 (zeros from K on).
+// The row prologue, in the arithmetic and order of the row kernel's one-wave rows (row_chain_kernel
+// with 64 threads, rowops.hip): lane t holds chunks c < CH of 8 elements at k = 8 * (64 c + t); the
+// sums of squares are added chunk by chunk, element by element, then across the wave by
+// wave_sum_dpp (chunks past K hold zeros, which change no sum).  It is latency, not throughput, that it costs: every workgroup makes the row again
+// while its weights are in flight.  So CH waves share it: each takes the sums over the whole row (a
+// multiply and an add per element) but the element-wise work, with its roundings, of chunk `wave`
+// only, and the chunks of h meet in LDS.  One wave doing all of it took the gate/up GEMV (K=1536,
+// N=12288) 3.9 us more than the plain GEMV's 6.65; see the figures at gemv1_launch.  Its operands
+// are fetched first (load), before the kernel issues its weight loads, so the arithmetic waits for
+// them alone; the row goes to xs [CH * 512] bf16 (zeros from K on), by way of hs [CH * 512].
 template <int CH>
 struct RowIn {
-  v4u y[CH], res[CH], w1[CH], w2[CH];
+  v4u y[CH], own, res, w1, w2;
   uint16_t scalar;
 
-  __device__ __forceinline__ void load(const GemvParams& p) {
+  __device__ __forceinline__ void load(const GemvParams& p, int wave) {
     const int t = threadIdx.x & 63;
-    scalar = p.pro_scalar ? *p.pro_scalar : uint16_t(0x3f80);
     const v4u one = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};  // bf16 1.0 x 8
+    const v4u zero = {0u, 0u, 0u, 0u};
+    scalar = p.pro_scalar ? *p.pro_scalar : uint16_t(0x3f80);
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
       const int k = 8 * (64 * c + t);
-      const bool in = k < p.K;
-      y[c] = in ? *reinterpret_cast<const v4u*>(p.pro_y + k) : v4u{0u, 0u, 0u, 0u};
-      res[c] = (in && p.pro_res) ? *reinterpret_cast<const v4u*>(p.pro_res + k) : v4u{0u, 0u, 0u, 0u};
-      w1[c] = (in && p.pro_w1) ? *reinterpret_cast<const v4u*>(p.pro_w1 + k) : one;
-      w2[c] = (in && p.pro_norm2 && p.pro_w2) ? *reinterpret_cast<const v4u*>(p.pro_w2 + k) : one;
+      y[c] = k < p.K ? *reinterpret_cast<const v4u*>(p.pro_y + k) : zero;
     }
+    const int k = 8 * (64 * wave + t);
+    const bool in = k < p.K;
+    own = in ? *reinterpret_cast<const v4u*>(p.pro_y + k) : zero;
+    res = (in && p.pro_res) ? *reinterpret_cast<const v4u*>(p.pro_res + k) : zero;
+    w1 = (in && p.pro_w1) ? *reinterpret_cast<const v4u*>(p.pro_w1 + k) : one;
+    w2 = (in && p.pro_norm2 && p.pro_w2) ? *reinterpret_cast<const v4u*>(p.pro_w2 + k) : one;
   }
 
-  // The values stay packed as bf16 between steps (every intermediate the row kernel rounds to bf16
-  // is exactly a bf16), which keeps the prologue's registers few while the weights are in flight.
-  __device__ __forceinline__ void make(const GemvParams& p, uint16_t* xs) {
-    const int t = threadIdx.x & 63, N = p.K;
+  // 1 / rms over the row whose chunks are in `c`.
+  __device__ __forceinline__ static float inv_rms(const v4u (&c)[CH], const GemvParams& p) {
     float ss = 0.0f;
 #pragma unroll
-    for (int c = 0; c < CH; ++c) {
+    for (int i = 0; i < CH; ++i) {
       float v[8];
-      unpack8(y[c], v);
+      unpack8(c[i], v);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) ss += v[i] * v[i];
+      for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
     }
     ss = wave_sum_dpp(ss);
-    const float r = 1.0f / sqrtf(ss / float(N) + p.pro_eps);
+    return 1.0f / sqrtf(ss / float(p.K) + p.pro_eps);
+  }
+
+  // This wave's chunk of h (wave < CH).
+  __device__ __forceinline__ v4u make_h(const GemvParams& p) const {
+    const float r = inv_rms(y, p);
     const float scl = bf16_to_f32(scalar);
+    float v[8], rv[8], wv[8];
+    unpack8(own, v);
+    unpack8(res, rv);
+    unpack8(w1, wv);
 #pragma unroll
-    for (int c = 0; c < CH; ++c) {
-      float v[8], rv[8], wv[8];
-      unpack8(y[c], v);
-      unpack8(res[c], rv);
-      unpack8(w1[c], wv);
+    for (int i = 0; i < 8; ++i) {
+      float n = v[i] * r;
+      if (p.pro_w1) n = n * wv[i];
+      v[i] = p.pro_res ? round_bf16(rv[i] + round_bf16(n)) : round_bf16(n);
+      if (p.pro_scalar) v[i] = round_bf16(v[i] * scl);
+    }
+    return pack8(v);
+  }
+
+  // Called by every wave of the workgroup; the row is whole in xs after the caller's barrier.
+  __device__ __forceinline__ void make(const GemvParams& p, int wave, uint16_t* xs, uint16_t* hs) {
+    const int t = threadIdx.x & 63;
+    const int k = 8 * (64 * wave + t);
+    v4u h = {0u, 0u, 0u, 0u};
+    if (wave < CH) {
+      h = make_h(p);
+      if (k >= p.K) h = v4u{0u, 0u, 0u, 0u};
+      if (p.pro_h && blockIdx.x == 0 && k < p.K) *reinterpret_cast<v4u*>(p.pro_h + k) = h;
+      *reinterpret_cast<v4u*>((p.pro_norm2 ? hs : xs) + k) = h;
+    }
+    if (!p.pro_norm2) return;
+    __syncthreads();
+    if (wave < CH) {
+      v4u hc[CH];
+#pragma unroll
+      for (int c = 0; c < CH; ++c) hc[c] = *reinterpret_cast<const v4u*>(hs + 8 * (64 * c + t));
+      const float r2 = inv_rms(hc, p);
+      float v[8], wv[8];
+      unpack8(h, v);
+      unpack8(w2, wv);
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        float n = v[i] * r;
-        if (p.pro_w1) n = n * wv[i];
-        v[i] = p.pro_res ? round_bf16(rv[i] + round_bf16(n)) : round_bf16(n);
-        if (p.pro_scalar) v[i] = round_bf16(v[i] * scl);
+        float n = v[i] * r2;
+        if (p.pro_w2) n = n * wv[i];
+        v[i] = round_bf16(n);
       }
-      y[c] = pack8(v);  // h
-    }
-    if (p.pro_h && blockIdx.x == 0) {
-#pragma unroll
-      for (int c = 0; c < CH; ++c) {
-        const int k = 8 * (64 * c + t);
-        if (k < N) *reinterpret_cast<v4u*>(p.pro_h + k) = y[c];
-      }
-    }
-    if (p.pro_norm2) {
-      float s2 = 0.0f;
-#pragma unroll
-      for (int c = 0; c < CH; ++c) {
-        float v[8];
-        unpack8(y[c], v);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) s2 += v[i] * v[i];
-      }
-      s2 = wave_sum_dpp(s2);
-      const float r2 = 1.0f / sqrtf(s2 / float(N) + p.pro_eps);
-#pragma unroll
-      for (int c = 0; c < CH; ++c) {
-        float v[8], wv[8];
-        unpack8(y[c], v);
-        unpack8(w2[c], wv);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          float n = v[i] * r2;
-          if (p.pro_w2) n = n * wv[i];
-          v[i] = round_bf16(n);
-        }
-        y[c] = pack8(v);
-      }
-    }
-#pragma unroll
-    for (int c = 0; c < CH; ++c) {
-      const int k = 8 * (64 * c + t);
-      *reinterpret_cast<v4u*>(xs + k) = k < N ? y[c] : v4u{0u, 0u, 0u, 0u};
+      *reinterpret_cast<v4u*>(xs + k) = k < p.K ? pack8(v) : v4u{0u, 0u, 0u, 0u};
     }
   }
 };
@@ -234,6 +249,92 @@ __device__ __forceinline__ v8bf widen8(uint32_t lo, uint32_t hi) {
   return __builtin_bit_cast(v8bf, r);
 }
 
+// k-block of 64 on the MFMA: 16 weight rows' bytes against the activation columns, added to acc.
+__device__ __forceinline__ v4f mma_block(v4i w, v4i xa, v4i xb, v4f acc) {
+  const v8bf wa = widen8(uint32_t(w[0]), uint32_t(w[1]));
+  const v8bf wb = widen8(uint32_t(w[2]), uint32_t(w[3]));
+  acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, __builtin_bit_cast(v8bf, xa), acc, 0, 0, 0);
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb, __builtin_bit_cast(v8bf, xb), acc, 0, 0, 0);
+}
+
+// 16 weight bytes; the packed stream with the streaming (sc0 nt) policy.
+template <bool PACKED>
+__device__ __forceinline__ v4i load_weight(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+  return __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, PACKED ? 3 : 0));
+}
+
+// The epilogue's operands of one lane: for T tiles `tstep` columns apart, the scales of columns n0 ..
+// n0+3, and for ACT 2 row m's multipliers.  load() only asks for them, bounds-checked and without a
+// branch or a conversion per element (either would wait for the element before the next is asked
+// for: 3 us of the gate/up GEMV); scale() and mul() convert.  Columns past N read zero and are not
+// stored.
+template <int T, int ACT>
+struct GemvScales {
+  uint32_t s[T][4], m[4];
+
+  __device__ __forceinline__ void load(const GemvParams& p, int row, int n0, int tstep) {
+    const __amdgpu_buffer_rsrc_t rs = make_rsrc(p.s, uint32_t(p.N) * (p.s_f32 ? 4u : 2u));
+    if (p.s_f32) {
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          s[t][r] = __builtin_amdgcn_raw_buffer_load_b32(rs, uint32_t(n0 + t * tstep + r) * 4u, 0, 0);
+    } else {
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          s[t][r] = __builtin_amdgcn_raw_buffer_load_b16(rs, uint32_t(n0 + t * tstep + r) * 2u, 0, 0);
+    }
+    if constexpr (ACT == 2) {
+      const __amdgpu_buffer_rsrc_t rm = make_rsrc(p.mul, uint32_t(((p.M - 1) * p.ldm + p.N) * 2));
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        m[r] = __builtin_amdgcn_raw_buffer_load_b16(rm, row < p.M ? uint32_t(row * p.ldm + n0 + r) * 2u : 0x80000000u, 0, 0);
+    }
+  }
+  __device__ __forceinline__ float scale(const GemvParams& p, int t, int r) const {
+    return __uint_as_float(p.s_f32 ? s[t][r] : s[t][r] << 16);
+  }
+  __device__ __forceinline__ float mul(int r) const { return __uint_as_float(m[r] << 16); }
+};
+
+__device__ __forceinline__ void store4(uint16_t* dst, const float (&o)[4], int n0, int n_end) {
+  if (n0 + 3 < n_end && ((reinterpret_cast<uintptr_t>(dst) & 7) == 0)) {
+    *reinterpret_cast<v2u*>(dst) = v2u{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
+  } else {
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (n0 + r < n_end) dst[r] = f32_to_bf16(o[r]);
+  }
+}
+
+// Row m, columns n0 .. n0+3 of tile t: y = bf16(acc * s).
+template <int T>
+__device__ __forceinline__ void store_plain(const GemvParams& p, const GemvScales<T, 0>& sc, int t, v4f acc, int m,
+                                            int n0) {
+  float o[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) o[r] = acc[r] * sc.scale(p, t, r);
+  store4(p.y + int64_t(m) * p.ldy + n0, o, n0, p.N);
+}
+
+// The bf16 GEMV outputs, then the activation with the row kernel's roundings: a, b the gate and up
+// sums (ACT 1), or a the gate's alone (ACT 2).
+template <int ACT, int T>
+__device__ __forceinline__ void store_act(const GemvParams& p, const GemvScales<T, ACT>& sc, v4f a, v4f b, int m, int n0) {
+  float o[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const float g = round_bf16(a[r] * sc.scale(p, 0, r));
+    const float u = ACT == 1 ? round_bf16(b[r] * sc.scale(p, T - 1, r)) : sc.mul(r);
+    o[r] = round_bf16(gelu_tanh_f32(g)) * u;
+  }
+  store4(p.y + int64_t(m) * p.ldy + n0, o, n0, ACT == 1 ? p.half_tiles * 16 : p.N);
+}
+
+// ---- 2..16 rows, and the LM head's many tiles ---------------------------------------------------
 // A wave multiplies TPW n-tiles of 16 weight rows against the M <= 16 activation rows: per k-block
 // of 64 it loads the activation fragment once and TPW weight fragments, and issues 2*TPW MFMAs.
 // With split > 1 the waves of a group take interleaved k-blocks and their partial sums are added
@@ -246,17 +347,17 @@ __device__ __forceinline__ v8bf widen8(uint32_t lo, uint32_t hi) {
 // LM head (K=1536, N=262144), 6.2 TB/s against 5.0 TB/s for the row-major weight, where each load
 // takes 64-byte pieces of 16 rows.  Row-major weights keep the default policy (a streamed half
 // line would be fetched twice).
-template <int TPW, int U, bool PACKED, int NWB, int ACT = 0, int PRO = 0>
+template <int TPW, int U, bool PACKED, int NWB, int ACT = 0>
 __global__ __launch_bounds__(NWB * 64) void gemv_kernel(GemvParams p) {
   static_assert(ACT != 1 || TPW == 2, "a GELU pair is one gate and one up tile per wave");
   __shared__ v4f red[NWB][TPW][64];
-  __shared__ __attribute__((aligned(16))) uint16_t xs[PRO == 4 ? 4096 : PRO ? PRO * 512 : 8];  // PRO: the row
-  __shared__ float mw[PRO == 4 ? 16 * (DEC_MERGE_IN_GEMV_CHUNKS + 1) : 1];     // PRO 4: chunk weights
   const int lane = threadIdx.x & 63;
-  const int wave = threadIdx.x >> 6;
-  const int group_in_block = wave / p.split;
-  const int ks = wave % p.split;
-  const int groups_per_block = NWB / p.split;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+  // 8 and 16 waves always share one tile group (gemv_launch_few)
+  const int split = NWB >= 8 ? NWB : p.split;
+  const int group_in_block = wave / split;
+  const int ks = wave % split;
+  const int groups_per_block = NWB / split;
   const int group = blockIdx.x * groups_per_block + group_in_block;
   // ACT 1: group g multiplies gate tile g and up tile g + half_tiles
   const int tile0 = ACT == 1 ? group : group * TPW;
@@ -268,6 +369,12 @@ __global__ __launch_bounds__(NWB * 64) void gemv_kernel(GemvParams p) {
   const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.x, p.x_bytes);
   const int kc = (lane >> 4) * 16;           // this lane's 16-byte chunk inside each 64-wide k-block
   const int mrow = lane & 15;                // activation row this lane supplies
+  // acc[t] of lane l holds row m = l % 16, columns (tile0 + t * tstride)*16 + ncol .. +3
+  const int ncol = 4 * (lane >> 4);
+  GemvScales<TPW, ACT> sc;
+  // few tiles: the epilogue's operands come with the weights, not a round trip after them
+  if (split > 1 && ks == 0 && active) sc.load(p, mrow, tile0 * 16 + ncol, tstride * 16);
+
   // Weight rows past N and activation rows past M start at or past the buffer ends and read 0.
   uint32_t wbase[TPW];
 #pragma unroll
@@ -275,76 +382,23 @@ __global__ __launch_bounds__(NWB * 64) void gemv_kernel(GemvParams p) {
     wbase[t] = PACKED ? uint32_t(tile0 + t * tstride) * uint32_t(p.KB) * 1024u + uint32_t(lane) * 16u
                       : uint32_t((tile0 + t * tstride) * 16 + (lane & 15)) * uint32_t(p.ldw) + uint32_t(kc);
   constexpr uint32_t W_KB = PACKED ? 1024u : 64u;  // weight bytes between k-blocks
-  constexpr int W_POL = PACKED ? 3 : 0;              // sc0 nt for the packed stream
   const uint32_t xbase = (uint32_t(mrow) * uint32_t(p.ldx) + uint32_t(kc)) * 2u;
 
   v4f acc[TPW];
 #pragma unroll
   for (int t = 0; t < TPW; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
-  // PRO: the activation row is made once per workgroup by its first wave (one row: M = 1) while
-  // every wave's first round of weight fragments is in flight.
-  RowIn<(PRO >= 1 && PRO <= 3) ? PRO : 1> row;
-  v4i wpre[U][TPW];
-  if constexpr (PRO) {
-    if (PRO <= 3 && wave == 0) row.load(p);
-    // Issued without branches (a fragment outside the weight is read past the buffer's end as
-    // zeros), so the prologue's arithmetic can wait for its own operands and leave these in flight.
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int kb = ks + u * p.split;
-      const bool ok = active && kb < p.KB && kb * 64 + kc < p.K;
-#pragma unroll
-      for (int t = 0; t < TPW; ++t)
-        wpre[u][t] = __builtin_bit_cast(
-            v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, ok ? wbase[t] + uint32_t(kb) * W_KB : 0x80000000u, 0, W_POL));
-    }
-    if constexpr (PRO == 4)
-      gemv_attn_merge_row(p, xs, mw);
-    else if (wave == 0)
-      row.make(p, xs);
-    __syncthreads();
-  }
   if (active) {
-    const int stride = p.split * U;
-    int kb0 = ks;
-    if constexpr (PRO) {
-      // the first round: its weights are in registers, the row in LDS
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int kb = kb0 + u * p.split;
-        v4i xa = {0, 0, 0, 0}, xb = {0, 0, 0, 0};
-        if (kb < p.KB && kb * 64 + kc < p.K && mrow == 0) {
-          const v4i* xv = reinterpret_cast<const v4i*>(xs + kb * 64 + kc);
-          xa = xv[0];
-          xb = xv[1];
-        }
-#pragma unroll
-        for (int t = 0; t < TPW; ++t) {
-          const v8bf wa = widen8(uint32_t(wpre[u][t][0]), uint32_t(wpre[u][t][1]));
-          const v8bf wb = widen8(uint32_t(wpre[u][t][2]), uint32_t(wpre[u][t][3]));
-          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa, __builtin_bit_cast(v8bf, xa), acc[t], 0, 0, 0);
-          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb, __builtin_bit_cast(v8bf, xb), acc[t], 0, 0, 0);
-        }
-      }
-      kb0 += stride;
-    }
-    for (; kb0 < p.KB; kb0 += stride) {
+    const int stride = split * U;
+    for (int kb0 = ks; kb0 < p.KB; kb0 += stride) {
       v4i wv[U][TPW], xa[U], xb[U];
 #pragma unroll
       for (int u = 0; u < U; ++u) {
-        const int kb = kb0 + u * p.split;
+        const int kb = kb0 + u * split;
         if (kb < p.KB && kb * 64 + kc < p.K) {
-          if constexpr (PRO) {
-            const v4i* xv = reinterpret_cast<const v4i*>(xs + kb * 64 + kc);
-            xa[u] = mrow == 0 ? xv[0] : v4i{0, 0, 0, 0};
-            xb[u] = mrow == 0 ? xv[1] : v4i{0, 0, 0, 0};
-          } else {
-            xa[u] = buf_load16(rx, xbase + uint32_t(kb) * 128u);
-            xb[u] = buf_load16(rx, xbase + uint32_t(kb) * 128u + 16u);
-          }
+          xa[u] = buf_load16(rx, xbase + uint32_t(kb) * 128u);
+          xb[u] = buf_load16(rx, xbase + uint32_t(kb) * 128u + 16u);
 #pragma unroll
-          for (int t = 0; t < TPW; ++t)
-            wv[u][t] = __builtin_bit_cast(v4i, __builtin_amdgcn_raw_buffer_load_b128(rw, wbase[t] + uint32_t(kb) * W_KB, 0, W_POL));
+          for (int t = 0; t < TPW; ++t) wv[u][t] = load_weight<PACKED>(rw, wbase[t] + uint32_t(kb) * W_KB);
         } else {
           xa[u] = v4i{0, 0, 0, 0};
           xb[u] = v4i{0, 0, 0, 0};
@@ -355,81 +409,199 @@ __global__ __launch_bounds__(NWB * 64) void gemv_kernel(GemvParams p) {
 #pragma unroll
       for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int t = 0; t < TPW; ++t) {
-          const v8bf w0 = widen8(uint32_t(wv[u][t][0]), uint32_t(wv[u][t][1]));
-          const v8bf w1 = widen8(uint32_t(wv[u][t][2]), uint32_t(wv[u][t][3]));
-          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w0, __builtin_bit_cast(v8bf, xa[u]), acc[t], 0, 0, 0);
-          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1, __builtin_bit_cast(v8bf, xb[u]), acc[t], 0, 0, 0);
-        }
+        for (int t = 0; t < TPW; ++t) acc[t] = mma_block(wv[u][t], xa[u], xb[u], acc[t]);
     }
   }
 
-  if (p.split > 1) {
+  const int m = lane & 15;
+  if (split > 1) {
+    // only the lanes of the M rows hold sums that are used
+    if (m < p.M) {
 #pragma unroll
-    for (int t = 0; t < TPW; ++t) red[wave][t][lane] = acc[t];
+      for (int t = 0; t < TPW; ++t) red[wave][t][lane] = acc[t];
+    }
     __syncthreads();
     if (ks != 0) return;
+    if (m < p.M) {
 #pragma unroll
-    for (int t = 0; t < TPW; ++t) {
-      acc[t] = red[wave][t][lane];
-      for (int q = 1; q < p.split; ++q) acc[t] += red[wave + q][t][lane];
+      for (int t = 0; t < TPW; ++t) {
+        acc[t] = red[wave][t][lane];
+        if constexpr (NWB >= 8) {
+          v4f part[NWB];
+#pragma unroll
+          for (int q = 1; q < NWB; ++q) part[q] = red[q][t][lane];
+#pragma unroll
+          for (int q = 1; q < NWB; ++q) acc[t] += part[q];
+        } else {
+          for (int q = 1; q < split; ++q) acc[t] += red[wave + q][t][lane];
+        }
+      }
     }
   }
-  if (!active) return;
-
-  // acc[t] lane l: row m = l % 16, columns n0 .. n0+3 with n0 = (tile0 + t)*16 + 4*(l/16).
-  const int m = lane & 15;
-  if (m >= p.M) return;
-  auto scale_at = [&](int nn) -> float {
-    return p.s_f32 ? reinterpret_cast<const float*>(p.s)[nn] : bf16_to_f32(reinterpret_cast<const uint16_t*>(p.s)[nn]);
-  };
+  if (!active || m >= p.M) return;
+  if (split == 1) sc.load(p, mrow, tile0 * 16 + ncol, tstride * 16);
   if constexpr (ACT != 0) {
-    // the bf16 GEMV outputs, then the activation with the row kernel's roundings
-    const int n0 = tile0 * 16 + 4 * (lane >> 4);
-    const int Nout = ACT == 1 ? p.half_tiles * 16 : p.N;
-    if (n0 >= Nout) return;
-    float o[4];
+    store_act<ACT>(p, sc, acc[0], acc[TPW - 1], m, tile0 * 16 + ncol);
+  } else {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int nn = n0 + r;
-      if (nn >= Nout) { o[r] = 0.0f; continue; }
-      const float g = round_bf16(acc[0][r] * scale_at(nn));
-      const float u = ACT == 1 ? round_bf16(acc[1][r] * scale_at(p.half_tiles * 16 + nn))
-                               : bf16_to_f32(p.mul[int64_t(m) * p.ldm + nn]);
-      o[r] = round_bf16(round_bf16(gelu_tanh_f32(g)) * u);
-    }
-    uint16_t* dst = p.y + int64_t(m) * p.ldy + n0;
-    if (n0 + 3 < Nout && ((reinterpret_cast<uintptr_t>(dst) & 7) == 0)) {
-      *reinterpret_cast<v2u*>(dst) = v2u{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
-    } else {
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (n0 + r < Nout) dst[r] = f32_to_bf16(o[r]);
-    }
-    return;
+    for (int t = 0; t < TPW; ++t) store_plain(p, sc, t, acc[t], m, (tile0 + t) * 16 + ncol);
   }
+}
+
+// ---- one row -------------------------------------------------------------------------------------
+// The decode step's linears (M = 1, 3-38 MB of weights).  They are bound by how many memory round
+// trips stand behind one another and by the busiest CU, not by HBM: a weight that lies in the cache
+// costs nearly what a cold one does.  So
+//  * everything the kernel will need is asked for at its start: the epilogue's scales and multiplier,
+//    the row's operands, then up to U fragments of weights per wave, all in flight while the row is
+//    made in LDS (PRO 3: the residual stream's norm, a row of 3 * 512; 4: the attention merge; 5:
+//    copied from x);
+//  * the tiles are dealt in units, `gpb` groups of `split` waves to a workgroup (gemv1_plan), and a
+//    wave multiplies no fragment past K: widening a KiB of bytes takes a SIMD about 130 clocks.
+// For the same reason a weight with few tiles (N = 1536: 96 of 16 rows on 256 CUs) is dealt in halves
+// (wide down 12288 x 1536: 9.6 us in whole tiles, 7.0 in halves): with HALF a unit is 8 weight rows, and a fragment load takes them from two
+// k-blocks at once: lane l holds row l % 8 of the unit, of k-block 2 q + (l % 16 >= 8) for pair q,
+// bytes 16 (l / 16).  The MFMA's column 0 gets the activations of the even k-block and column 1
+// those of the odd one, so the sums of rows 0..7 of column 0 and rows 8..15 of column 1 are the
+// unit's two parts, added first when the waves' partials are.  Without HALF, a GELU pair (ACT 1) is
+// 8 gate rows and the same 8 up rows in one tile, from the two fragments that hold them.
+// The order of every sum follows from (N, K) alone, so the plain GEMV, the activations and the
+// prologues agree bit for bit.
+template <int U, bool PACKED, int ACT, int PRO, bool HALF>
+__global__ __launch_bounds__(768) void gemv1_kernel(GemvParams p) {
+  constexpr bool NORM = PRO <= 3;                  // PRO chunks of 512 (K <= 1536)
+  constexpr int XS = PRO == 5 ? GEMV_ROW_MAX : PRO == 4 ? 4096 : PRO * 512;
+  constexpr int TPW = ACT == 1 && HALF ? 2 : 1;    // HALF pairs: the gate rows' and the up rows' fragments
+  constexpr bool SPLIT_ROWS = HALF || ACT == 1;    // a unit is 8 output columns
+  constexpr bool PAIR = ACT == 1 && !HALF;         // gate and up rows in one fragment
+  __shared__ v4f red[16][TPW][4];                  // per wave: rows 4j .. 4j+3 of its tile
+  __shared__ __attribute__((aligned(16))) uint16_t xs[XS];                    // the row
+  __shared__ __attribute__((aligned(16))) uint16_t hs[NORM ? PRO * 512 : 8];  // NORM: the first norm's row
+  __shared__ float mw[PRO == 4 ? MERGE_HEADS * (DEC_MERGE_IN_GEMV_CHUNKS + 1) : 1];  // PRO 4: chunk weights
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6);
+  const int split = p.split;
+  const int gib = wave / split, ks = wave % split;
+  const int unit = int(blockIdx.x) * p.gpb + gib;
+  const bool active = gib < p.gpb && unit < p.units;
+  const int i = lane & 15, j = lane >> 4;  // fragment row and 16-byte chunk
+
+  const __amdgpu_buffer_rsrc_t rw = make_rsrc(p.w, p.w_bytes);
+  const __amdgpu_buffer_rsrc_t rx = make_rsrc(p.x, p.x_bytes);
+  constexpr uint32_t PAST = 0x80000000u;  // an offset past every buffer here: reads zero
+
+  RowIn<NORM ? PRO : 1> row;
+  if constexpr (NORM) {
+    if (wave < PRO) row.load(p, wave);
+  }
+  // The epilogue runs on the group's first wave, lanes 16 j: columns n0 .. n0+3.
+  const int n0 = SPLIT_ROWS ? unit * 8 + 4 * j : unit * 16 + 4 * j;
+  GemvScales<ACT == 1 ? 2 : 1, ACT> sc;
+  if (ks == 0 && active) sc.load(p, i, n0, p.half_tiles * 16);
+
+  // Byte offset of this lane's piece of fragment t at k-block 0, and k-blocks between fragments.
+  const int sub = SPLIT_ROWS ? 8 * (unit & 1) + (i & 7) : i;  // row inside its 16-row tile
+  uint32_t wbase[TPW];
 #pragma unroll
   for (int t = 0; t < TPW; ++t) {
-    const int n0 = (tile0 + t) * 16 + 4 * (lane >> 4);
-    if (n0 >= p.N) continue;
-    float o[4];
+    int tile = SPLIT_ROWS ? unit >> 1 : unit;
+    if (PAIR && i >= 8) tile += p.half_tiles;
+    if (TPW == 2 && t == 1) tile += p.half_tiles;
+    wbase[t] = PACKED ? uint32_t(tile) * uint32_t(p.KB) * 1024u + uint32_t(j * 16 + sub) * 16u
+                      : uint32_t(tile * 16 + sub) * uint32_t(p.ldw) + uint32_t(j * 16);
+  }
+  constexpr uint32_t W_KB = PACKED ? 1024u : 64u;  // weight bytes between k-blocks
+  const int nstep = HALF ? (p.KB + 1) >> 1 : p.KB;   // steps over K: pairs of k-blocks with HALF
+  const int hi = HALF ? i >> 3 : 0;                  // this lane's weight k-block within its pair
+  auto load_w = [&](int st, v4i (&w)[TPW]) {
+    const int kb = HALF ? 2 * st + hi : st;
+    const bool ok = active && kb < p.KB && kb * 64 + j * 16 < p.K;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int nn = n0 + r;
-      float sc = 0.0f;
-      if (nn < p.N) sc = p.s_f32 ? reinterpret_cast<const float*>(p.s)[nn]
-                                 : bf16_to_f32(reinterpret_cast<const uint16_t*>(p.s)[nn]);
-      o[r] = acc[t][r] * sc;
+    for (int t = 0; t < TPW; ++t) w[t] = load_weight<PACKED>(rw, ok ? wbase[t] + uint32_t(kb) * W_KB : PAST);
+  };
+
+  v4i wv[U][TPW];
+  if constexpr (PRO == 5) {
+    // The row's pieces of 8 are asked for before the weights, two per thread (all of it from 12 waves
+    // on); a wait inside a loop would be one for the weights too.
+    const int k0 = int(threadIdx.x) * 8, nt8 = int(blockDim.x) * 8, k1 = k0 + nt8;
+    for (int k = k1 + nt8; k < p.KB * 64; k += nt8)
+      *reinterpret_cast<v4i*>(xs + k) = buf_load16(rx, k < p.K ? uint32_t(k) * 2u : PAST);
+    const v4i x0 = buf_load16(rx, k0 < p.K ? uint32_t(k0) * 2u : PAST);
+    const v4i x1 = buf_load16(rx, k1 < p.K ? uint32_t(k1) * 2u : PAST);
+#pragma unroll
+    for (int u = 0; u < U; ++u) load_w(ks + u * split, wv[u]);
+    if (k0 < p.KB * 64) *reinterpret_cast<v4i*>(xs + k0) = x0;
+    if (k1 < p.KB * 64) *reinterpret_cast<v4i*>(xs + k1) = x1;
+  } else {
+#pragma unroll
+    for (int u = 0; u < U; ++u) load_w(ks + u * split, wv[u]);
+    if constexpr (PRO == 4)
+      gemv_attn_merge_row(p, xs, mw);
+    else
+      row.make(p, wave, xs, hs);
+  }
+  __syncthreads();
+
+  v4f acc[TPW];
+#pragma unroll
+  for (int t = 0; t < TPW; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int st0 = ks; st0 < nstep; st0 += split * U) {
+    if (st0 != ks) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) load_w(st0 + u * split, wv[u]);
     }
-    uint16_t* dst = p.y + int64_t(m) * p.ldy + n0;
-    if (n0 + 3 < p.N && ((reinterpret_cast<uintptr_t>(dst) & 7) == 0)) {
-      *reinterpret_cast<v2u*>(dst) = v2u{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
-    } else {
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (n0 + r < p.N) dst[r] = f32_to_bf16(o[r]);
+    for (int u = 0; u < U; ++u) {
+      // activation column i: with HALF column 0 takes the even k-block, column 1 the odd one
+      const int st = st0 + u * split;
+      if (st >= nstep) break;
+      const int kb = HALF ? 2 * st + i : st;
+      v4i xa = {0, 0, 0, 0}, xb = {0, 0, 0, 0};
+      if (i < (HALF ? 2 : 1) && kb < p.KB && kb * 64 + j * 16 < p.K) {
+        const v4i* xv = reinterpret_cast<const v4i*>(xs + kb * 64 + j * 16);
+        xa = xv[0];
+        xb = xv[1];
+      }
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) acc[t] = mma_block(wv[u][t], xa, xb, acc[t]);
     }
   }
+
+  // Partials: lane 16 j + c holds rows 4j .. 4j+3 of column c; HALF's rows 8.. belong to column 1.
+  if (i == (HALF && j >= 2 ? 1 : 0)) {
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) red[wave][t][j] = acc[t];
+  }
+  __syncthreads();
+  if (ks != 0 || !active) return;
+  // Lanes 16 j add the group's partials of rows 4j .. wave by wave; lanes 0 and 16 then take rows 8..
+  // (with HALF the same columns' other part, in a PAIR their up sums) from lanes 32 and 48.
+  v4f sum[TPW], other[TPW];
+#pragma unroll
+  for (int t = 0; t < TPW; ++t) {
+    // sixteen reads without a branch; those past the group are another wave's and left out
+    v4f part[16];
+#pragma unroll
+    for (int q = 0; q < 16; ++q) part[q] = red[(wave + q) & 15][t][j];
+    sum[t] = part[0];
+#pragma unroll
+    for (int q = 1; q < 16; ++q) {
+      const v4f s = sum[t] + part[q];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) sum[t][r] = q < split ? s[r] : sum[t][r];
+    }
+    if constexpr (SPLIT_ROWS) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) other[t][r] = __shfl_xor(sum[t][r], 32, 64);
+      if constexpr (HALF) sum[t] += other[t];
+    }
+  }
+  if (i != 0 || (SPLIT_ROWS && j >= 2)) return;
+  if constexpr (ACT == 0)
+    store_plain(p, sc, 0, sum[0], 0, n0);
+  else
+    store_act<ACT>(p, sc, sum[0], PAIR ? other[0] : sum[TPW - 1], 0, n0);
 }
 
 // Row-major int8 W [N, K] (ld = ldw) -> GEMV fragment layout, one thread per 16-byte piece;
@@ -470,9 +642,83 @@ static int few_tile_split(int64_t ntiles, int KB) {
   return split;
 }
 
+// The few-tile launch of 2..16 rows: per tile group `split` waves, NWB = split for 8 and 16.
+template <bool PACKED, int TPW, int ACT>
+static void gemv_launch_few(const GemvParams& p, int64_t groups, hipStream_t stream) {
+  const int per_wave = (p.KB + p.split - 1) / p.split;
+  if (p.split <= 4) {
+    const int gpb = 4 / p.split;
+    gemv_kernel<TPW, 4, PACKED, 4, ACT><<<unsigned((groups + gpb - 1) / gpb), 256, 0, stream>>>(p);
+  } else if (p.split == 8) {
+    gemv_kernel<TPW, 4, PACKED, 8, ACT><<<unsigned(groups), 512, 0, stream>>>(p);
+  } else if (per_wave > 4 && per_wave <= 6) {
+    // five or six k-blocks per wave (the down projection, K=6144): all of them in one round
+    // trip instead of two
+    gemv_kernel<TPW, 6, PACKED, 16, ACT><<<unsigned(groups), 1024, 0, stream>>>(p);
+  } else {
+    gemv_kernel<TPW, 4, PACKED, 16, ACT><<<unsigned(groups), 1024, 0, stream>>>(p);
+  }
+}
+
+// One row: HALF where the 16-row tiles would leave half of the CUs without one.  A unit's K range is
+// split over 8 waves while a CU has one unit (HALF, or N <= 4096 on 256 CUs), over 4 from two units
+// per CU on: the waves of a CU then stand evenly on its four SIMDs (3 or 6 waves per unit cost the
+// gate/up GEMV 1-2 us more), and more waves only add partials (down 6144 x 1536 in halves: 16 waves
+// 5.5 us, 8 waves 4.8, 6 waves 5.5).  The split depends on (N, K) alone; the units per
+// workgroup, which change no sum, are one, or with a row to make (the norm, the merge) up to three,
+// so that the row is made less often (gate/up 1536 x 12288: 8.4 us with one, 7.5 with three).
+static bool gemv1_plan(GemvParams& p, bool make_row) {
+  const int cus = gemv_cu_count();
+  const int ntiles = (p.N + 15) / 16;
+  const bool half = 2 * ntiles <= cus;
+  const int per_cu = half ? 1 : (ntiles + cus - 1) / cus;
+  p.units = half ? (p.N + 7) / 8 : ntiles;
+  p.split = min(per_cu == 1 ? 8 : 4, half ? (p.KB + 1) / 2 : p.KB);
+  p.gpb = make_row ? min(per_cu, 3) : 1;
+  return half;
+}
+
+// Whether a call takes the one-row kernel: its row fits in LDS and its tiles are few.
+static bool gemv1_takes(const GemvParams& p) {
+  return p.M == 1 && p.KB * 64 <= GEMV_ROW_MAX && (int64_t(p.N) + 15) / 16 < 4096;
+}
+
+// U fragments in flight per wave: all of a wave's share in one round where the registers allow it.
+// MI355X, weights cold, a chain of launches replayed from a graph (a chain of empty ones takes 1.9 us
+// each), us per launch, before (one tile per workgroup of 8 or 16 waves, the row made by one wave, the
+// scales fetched after the sums) -> now: o 2048 x 1536 4.5 -> 3.6, 4096 x 1536 5.5 -> 4.2; qkv 1536 x
+// 2560 with its norm 6.3 -> 4.8; gate/up with norm and GELU 1536 x 12288 10.6 -> 7.7, x 24576 13.8 ->
+// 12.1; down 6144 x 1536 7.0 -> 5.0, 12288 x 1536 10.5 -> 7.0; per-layer gate 1536 x 256 with norm
+// 6.3 -> 4.6, projection 256 x 1536 3.3 -> 3.0.
+template <bool PACKED, int ACT, int PRO>
+static void gemv1_launch(const GemvParams& p0, hipStream_t stream) {
+  GemvParams p = p0;
+  // ACT 1 deals the same number of units of 8 gate and 8 up rows as the plain launch of N has
+  // tiles, so its sums are made in the same order
+  const bool half = gemv1_plan(p, PRO != 5);
+  if (ACT == 1 && half) p.units = (p.N / 2 + 7) / 8;
+  const int waves = max(p.gpb * p.split, PRO <= 3 ? PRO : 1);  // the norm's chunks each need a wave
+  const dim3 grid(unsigned((p.units + p.gpb - 1) / p.gpb)), block(unsigned(waves * 64));
+  const int steps = half ? (p.KB + 1) / 2 : p.KB;
+  const int per_wave = (steps + p.split - 1) / p.split;
+#define W8A8_GEMV1(U)                                                                   \
+  do {                                                                                  \
+    if (half) gemv1_kernel<U, PACKED, ACT, PRO, true><<<grid, block, 0, stream>>>(p);   \
+    else gemv1_kernel<U, PACKED, ACT, PRO, false><<<grid, block, 0, stream>>>(p);       \
+  } while (0)
+  if (per_wave <= 1) W8A8_GEMV1(1);
+  else if (per_wave <= 2) W8A8_GEMV1(2);
+  else if (per_wave <= 3) W8A8_GEMV1(3);
+  else if (per_wave <= 4 || (ACT == 1 && half)) W8A8_GEMV1(4);
+  else if (per_wave <= 6 || half || PRO == 4) W8A8_GEMV1(6);
+  else gemv1_kernel<PRO == 4 ? 6 : 12, PACKED, ACT, PRO, false><<<grid, block, 0, stream>>>(p);
+#undef W8A8_GEMV1
+}
+
 template <bool PACKED>
 static void gemv_launch(const GemvParams& p0, hipStream_t stream) {
   GemvParams p = p0;
+  if (gemv1_takes(p)) return gemv1_launch<PACKED, 0, 5>(p, stream);
   const int64_t ntiles = (p.N + 15) / 16;
   if (ntiles >= 4096) {
     // Many n-tiles (the LM head): each activation fragment serves two (M <= 8) or four
@@ -485,52 +731,26 @@ static void gemv_launch(const GemvParams& p0, hipStream_t stream) {
       const int64_t groups = (ntiles + 3) / 4;
       gemv_kernel<4, 2, PACKED, 4><<<unsigned((groups + 3) / 4), 256, 0, stream>>>(p);
     }
-  } else {
-    // Few n-tiles (the per-layer decode shapes: 96-768 tiles): one tile per group of `split`
-    // waves that share its K range, up to 16 waves of one workgroup, aiming for ~4096 waves over
-    // the chip's 1024 SIMDs, each with at least two k-blocks.  The weights here are 3-19 MB, so
-    // what bounds them is how many bytes are in flight: with at most four waves per tile the
-    // down projection (96 tiles) ran 384 waves and reached ~1 TB/s.
-    const int split = few_tile_split(ntiles, p.KB);
-    p.split = split;
-    if (split <= 4) {
-      const int gpb = 4 / split;
-      gemv_kernel<1, 4, PACKED, 4><<<unsigned((ntiles + gpb - 1) / gpb), 256, 0, stream>>>(p);
-    } else if (split == 8) {
-      gemv_kernel<1, 4, PACKED, 8><<<unsigned(ntiles), 512, 0, stream>>>(p);
-    } else if ((p.KB + 15) / 16 > 4 && (p.KB + 15) / 16 <= 6) {
-      // five or six k-blocks per wave (the down projection, K=6144): all of them in one round
-      // trip instead of two (M=1 cold token 837 -> 826 us)
-      gemv_kernel<1, 6, PACKED, 16><<<unsigned(ntiles), 1024, 0, stream>>>(p);
-    } else {
-      gemv_kernel<1, 4, PACKED, 16><<<unsigned(ntiles), 1024, 0, stream>>>(p);
-    }
+    return;
   }
+  // Few n-tiles (the per-layer decode shapes: 96-768 tiles): one tile per group of `split`
+  // waves that share its K range, up to 16 waves of one workgroup, aiming for ~4096 waves over
+  // the chip's 1024 SIMDs, each with at least two k-blocks.
+  p.split = few_tile_split(ntiles, p.KB);
+  gemv_launch_few<PACKED, 1, 0>(p, ntiles, stream);
 }
 
-// The few-tile launch with an activation epilogue: ACT 1 over I / 16 gate/up tile pairs (two tiles
-// per wave), ACT 2 over the N / 16 tiles.  The split and the unroll depth are the plain launch's
-// for the whole N (gemv_launch), so every tile's sum is added in the same order and the result is
-// the plain GEMV's, bit for bit, before the activation.  ACT 0 is the plain few-tile launch; PRO
-// (1..3, the prologue row's chunks per lane) adds the row prologue.
-template <bool PACKED, int ACT, int PRO = 0>
+// The packed few-tile launch with an activation epilogue: ACT 1 over I / 16 gate/up tile pairs (two
+// tiles per wave), ACT 2 over the N / 16 tiles.  The split is the plain launch's for the whole N, so
+// every tile's sum is added in the same order and the result is the plain GEMV's, bit for bit,
+// before the activation.
+template <int ACT>
 static void gemv_launch_act(const GemvParams& p0, hipStream_t stream) {
   GemvParams p = p0;
+  if (gemv1_takes(p)) return gemv1_launch<true, ACT, 5>(p, stream);
   const int64_t ntiles = (p.N + 15) / 16;
-  const int64_t groups = ACT == 1 ? p.half_tiles : ntiles;
-  const int split = few_tile_split(ntiles, p.KB);
-  p.split = split;
-  constexpr int TPW = ACT == 1 ? 2 : 1;
-  if (split <= 4) {
-    const int gpb = 4 / split;
-    gemv_kernel<TPW, 4, PACKED, 4, ACT, PRO><<<unsigned((groups + gpb - 1) / gpb), 256, 0, stream>>>(p);
-  } else if (split == 8) {
-    gemv_kernel<TPW, 4, PACKED, 8, ACT, PRO><<<unsigned(groups), 512, 0, stream>>>(p);
-  } else if (!PRO && (p.KB + 15) / 16 > 4 && (p.KB + 15) / 16 <= 6) {  // K > 4096: never with the prologue
-    gemv_kernel<TPW, 6, PACKED, 16, ACT, 0><<<unsigned(groups), 1024, 0, stream>>>(p);
-  } else {
-    gemv_kernel<TPW, 4, PACKED, 16, ACT, PRO><<<unsigned(groups), 1024, 0, stream>>>(p);
-  }
+  p.split = few_tile_split(ntiles, p.KB);
+  gemv_launch_few<true, ACT == 1 ? 2 : 1, ACT>(p, ACT == 1 ? p.half_tiles : ntiles, stream);
 }
 
 }  // namespace w8a8
@@ -604,9 +824,9 @@ extern "C" int w8a8_gemv_packed_act_bf16(const uint16_t* x, int64_t ldx, int64_t
   p.M = int(M); p.N = int(N); p.K = int(K); p.KB = int((K + 63) / 64);
   p.mul = mul; p.ldm = ldm; p.half_tiles = int(N / 32);
   if (act == 1)
-    gemv_launch_act<true, 1>(p, stream);
+    gemv_launch_act<1>(p, stream);
   else
-    gemv_launch_act<true, 2>(p, stream);
+    gemv_launch_act<2>(p, stream);
   return check_launch("gemv_packed_act_bf16");
 }
 
@@ -650,18 +870,9 @@ extern "C" int w8a8_gemv_packed_norm_bf16(const uint16_t* y, const uint16_t* res
   p.mul = mul; p.ldm = N; p.half_tiles = int(N / 32);
   p.pro_y = y; p.pro_res = res; p.pro_w1 = w1; p.pro_scalar = scalar; p.pro_w2 = w2; p.pro_h = h;
   p.pro_eps = eps; p.pro_norm2 = norm2 ? 1 : 0;
-  // the row kernel's chunks of 8 per lane for a row of K (K <= 1536: one wave, at most three)
-  p.pro_ch = int((K + 511) / 512);
-#define W8A8_NORM_GEMV(CH)                                                   \
-  do {                                                                       \
-    if (act == 0) gemv_launch_act<true, 0, CH>(p, stream);                   \
-    else if (act == 1) gemv_launch_act<true, 1, CH>(p, stream);              \
-    else gemv_launch_act<true, 2, CH>(p, stream);                            \
-  } while (0)
-  if (p.pro_ch == 1) W8A8_NORM_GEMV(1);
-  else if (p.pro_ch == 2) W8A8_NORM_GEMV(2);
-  else W8A8_NORM_GEMV(3);
-#undef W8A8_NORM_GEMV
+  if (act == 0) gemv1_launch<true, 0, 3>(p, stream);
+  else if (act == 1) gemv1_launch<true, 1, 3>(p, stream);
+  else gemv1_launch<true, 2, 3>(p, stream);
   return check_launch("gemv_packed_norm_bf16");
 }
 
@@ -698,7 +909,7 @@ extern "C" int w8a8_gemv_packed_attn_merge_bf16(const void* workspace, const int
   p.m_pos = q_pos; p.m_window = int(window); p.m_nchunk_grid = nchunk_grid; p.m_G = G; p.m_D = int(D);
   p.m_chunk = dec_chunk(int(D));
   p.m_c = scale * 1.4426950408889634f;  // the attention's exp2 factor, computed as it computes it
-  gemv_launch_act<true, 0, 4>(p, stream);
+  gemv1_launch<true, 0, 4>(p, stream);
   return check_launch("gemv_packed_attn_merge_bf16");
 }
 

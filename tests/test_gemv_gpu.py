@@ -309,3 +309,49 @@ def test_gemv_norm_refusals():
     head = ops.pack_gemv_weight(torch.ones((65536, K), dtype=torch.int8, device=dev))
     with pytest.raises(W8A8Error, match="few-tile"):
         ops.gemv_norm_bf16(y, None, w1, 1e-6, head, torch.ones(65536, device=dev).to(torch.bfloat16))
+
+
+# One row: N at the edges of the unit plan on 256 CUs (halves of tiles up to 2048, one tile per CU up to
+# 4096, then several; N no multiple of 16 or 8), K at odd counts of k-blocks, ragged last k-blocks,
+# fewer steps than waves, the longest row held in LDS and the first beyond it.
+ONE_ROW = [(1536, 16), (1536, 64), (1536, 80), (8, 1536), (2040, 1552), (2048, 192), (2064, 192), (2049, 80),
+           (4096, 320), (4112, 320), (8200, 272), (12288, 96), (24576, 64), (65520, 48), (40, 12288), (1536, 12288),
+           (2064, 12288), (40, 12304)]
+
+
+@pytest.mark.parametrize("N, K", ONE_ROW)
+def test_gemv_one_row_exact_at_the_plan_edges(N, K):
+    """Integer activations: every partial sum is an integer below 2^24, so the one-row GEMV equals
+    bf16(product * s) whatever its split, packed and row-major, bf16 and fp32 scales."""
+    g = torch.Generator(device=DEV).manual_seed(N * 7 + K)
+    x = torch.randint(-3, 4, (1, K), generator=g, device=DEV)
+    w = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8, device=DEV)
+    acc = (x.double() @ w.double().t()).float()
+    print(f"one-row GEMV N={N} K={K}", flush=True)
+    for s in (torch.rand(N, generator=g, device=DEV) * 0.01 + 0.005,
+              (torch.rand(N, generator=g, device=DEV) * 0.01 + 0.005).to(torch.bfloat16)):
+        ref = (acc * s.float()[None, :]).to(torch.bfloat16)
+        xb = x.to(torch.bfloat16)
+        assert torch.equal(ops.gemv_bf16(xb, ops.pack_gemv_weight(w), s), ref)
+        assert torch.equal(ops.gemv_bf16(xb, w, s), ref)
+
+
+@pytest.mark.parametrize("I, K", [(16, 64), (48, 1536), (1024, 1536), (1040, 320), (6144, 80), (4096, 12288)])
+def test_gemv_one_row_gelu_pair_and_norm_agree(I, K):
+    """The pair's units (halves of both tiles up to N = 2I = 2048, gate and up rows in one tile beyond)
+    and the norm prologue against the plain one-row GEMV and the row kernels, bit for bit."""
+    g = torch.Generator(device=DEV).manual_seed(I + K)
+    w = torch.randint(-127, 128, (2 * I, K), generator=g, dtype=torch.int8, device=DEV)
+    pw = ops.pack_gemv_weight(w)
+    s = torch.rand(2 * I, generator=g, device=DEV) * 0.01
+    y, r = (torch.randn(1, K, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
+    w1, w2 = ((1 + 0.1 * torch.randn(K, generator=g, device=DEV)).to(torch.bfloat16) for _ in range(2))
+    print(f"one-row pair I={I} K={K}", flush=True)
+    assert torch.equal(ops.gemv_act_bf16(y, pw, s, "gelu_pair"), ops.gelu_mul_bf16(ops.gemv_bf16(y, pw, s)))
+    if K > 1536:
+        return
+    h, x = ops.rms_residual_norm(y, r, w1, w2, 1e-6)
+    got, gh = ops.gemv_norm_bf16(y, r, w1, 1e-6, pw, s, act="gelu_pair", w2=w2)
+    assert torch.equal(gh, h) and torch.equal(got, ops.gelu_mul_bf16(ops.gemv_bf16(x, pw, s)))
+    got, _ = ops.gemv_norm_bf16(y, r, w1, 1e-6, pw, s, w2=w2)
+    assert torch.equal(got, ops.gemv_bf16(x, pw, s))
