@@ -159,35 +159,29 @@ __device__ __forceinline__ void attn_quant_tokens(const AttnParams& p, const cha
     a = *reinterpret_cast<const v4u*>(src);
     b = *reinterpret_cast<const v4u*>(src + 16);
   };
-  float amax = 0.0f;
+  uint32_t m2 = 0;
   if (live)
     for (int c = j; c < NCH; c += TPT) {
       v4u a, b;
       chunk(c, a, b);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        amax = absmax2(amax, absmax2(fabsf(__uint_as_float(a[e] << 16)), fabsf(__uint_as_float(a[e] & 0xffff0000u))));
-        amax = absmax2(amax, absmax2(fabsf(__uint_as_float(b[e] << 16)), fabsf(__uint_as_float(b[e] & 0xffff0000u))));
-      }
+      for (int e = 0; e < 4; ++e) m2 = absmax_bf16x2(absmax_bf16x2(m2, a[e]), b[e]);
     }
+  float amax = absmax_pair(m2);
   for (int o = 1; o < TPT; o <<= 1) amax = absmax2(amax, __shfl_xor(amax, o, 64));
   const float s = quant_scale(amax);
   const float rs = 1.0f / s;
   if (live) {
     if (j == 0) p.qsx[t] = s;
+    const bool finite = quant_finite(s);
     for (int c = j; c < NCH; c += TPT) {
       v4u h[2];
       chunk(c, h[0], h[1]);
-      uint32_t w[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-      for (int hh = 0; hh < 2; ++hh)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const uint32_t lo = uint8_t(quant1_bf16(__uint_as_float(h[hh][e] << 16), s, rs));
-          const uint32_t hi = uint8_t(quant1_bf16(__uint_as_float(h[hh][e] & 0xffff0000u), s, rs));
-          w[2 * hh + (e >> 1)] |= (lo | (hi << 8)) << (16 * (e & 1));
-        }
-      *reinterpret_cast<v4u*>(p.qpk + packed_act_offset(t, 16 * c, p.qKF)) = v4u{w[0], w[1], w[2], w[3]};
+      float f0[8], f1[8];
+      unpack8(h[0], f0);
+      unpack8(h[1], f1);
+      const v2u lo = quant8(f0, s, rs, finite), hi = quant8(f1, s, rs, finite);
+      *reinterpret_cast<v4u*>(p.qpk + packed_act_offset(t, 16 * c, p.qKF)) = v4u{lo[0], lo[1], hi[0], hi[1]};
     }
   }
   if (tile == p.ntiles - 1)

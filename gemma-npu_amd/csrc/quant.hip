@@ -219,33 +219,26 @@ __global__ __launch_bounds__(256) void quant_rows_blk_kernel(const uint16_t* __r
     const int k = 8 * (256 * c + t);
     v[c] = k < K ? *reinterpret_cast<const v4u*>(xr + k) : v4u{0u, 0u, 0u, 0u};
   }
-  float amax = 0.0f;
+  uint32_t m2 = 0;
 #pragma unroll
   for (int c = 0; c < CH; ++c)
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      amax = absmax2(amax, absmax2(fabsf(__uint_as_float(v[c][i] << 16)), fabsf(__uint_as_float(v[c][i] & 0xffff0000u))));
-  amax = wave_absmax_dpp(amax);
+    for (int i = 0; i < 4; ++i) m2 = absmax_bf16x2(m2, v[c][i]);
+  float amax = wave_absmax_dpp(absmax_pair(m2));
   if ((t & 63) == 0) wave_amax[t >> 6] = amax;
   __syncthreads();
   amax = absmax2(absmax2(wave_amax[0], wave_amax[1]), absmax2(wave_amax[2], wave_amax[3]));
   const float s = quant_scale(amax);
   const float rs = 1.0f / s;
   if (t == 0) scale[row] = s;
+  const bool finite = quant_finite(s);
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
     const int k = 8 * (256 * c + t);
     if (k >= KP) continue;
-    uint32_t w[2] = {0u, 0u};
-    if (k < K) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const uint32_t lo = uint8_t(quant1_bf16(__uint_as_float(v[c][i] << 16), s, rs));
-        const uint32_t hi = uint8_t(quant1_bf16(__uint_as_float(v[c][i] & 0xffff0000u), s, rs));
-        w[i >> 1] |= (lo | (hi << 8)) << (16 * (i & 1));
-      }
-    }
-    *reinterpret_cast<v2u*>(dst(k)) = v2u{w[0], w[1]};
+    float f[8];
+    unpack8(v[c], f);  // past K the row was read as zeros, whose codes are zero
+    *reinterpret_cast<v2u*>(dst(k)) = quant8(f, s, rs, finite);
   }
 }
 
@@ -281,7 +274,7 @@ __global__ __launch_bounds__(256) void pack_act_kernel(const int8_t* __restrict_
   *reinterpret_cast<v4u*>(out + c * 16) = v;
 }
 
-// Self-check of quant1_bf16 against the IEEE-division form: one block per positive finite bf16
+// Self-check of quant1_bf16 and quant_bits against the IEEE-division form: one block per positive finite bf16
 // absmax a, its threads walking every bf16 v with |v| <= a.  counts[0] += pairs whose int8 codes
 // differ, counts[1] += pairs compared (1,065,402,240 in all).
 __global__ __launch_bounds__(256) void selfcheck_quant_step_kernel(unsigned long long* counts) {
@@ -293,7 +286,7 @@ __global__ __launch_bounds__(256) void selfcheck_quant_step_kernel(unsigned long
     const float v = bf16_to_f32(uint16_t(vh));
     if (!(fabsf(v) <= a)) continue;
     ++n;
-    bad += quant1_bf16(v, s, rs) != quant1(v, s);
+    bad += quant1_bf16(v, s, rs) != quant1(v, s) || int8_t(quant_bits(v, s, rs)) != quant1(v, s);
   }
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {

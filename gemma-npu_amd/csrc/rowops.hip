@@ -232,16 +232,12 @@ __global__ __launch_bounds__(256) void row_chain_kernel(RowChain p) {
   const float s = quant_scale(amax);
   const float rs = 1.0f / s;
   if (t == 0) p.sq[row] = s;
+  const bool finite = quant_finite(s);
 #pragma unroll
   for (int c = 0; c < CH; ++c) {
     const int k = 8 * (nt * c + t);
     if (k >= KQ) continue;
-    uint32_t w[2] = {0u, 0u};
-    if (k < p.N) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) w[i >> 2] |= uint32_t(uint8_t(quant1_bf16(v[c][i], s, rs))) << (8 * (i & 3));
-    }
-    *reinterpret_cast<v2u*>(qdst(k)) = v2u{w[0], w[1]};
+    *reinterpret_cast<v2u*>(qdst(k)) = k < p.N ? quant8(v[c], s, rs, finite) : v2u{0u, 0u};
   }
 }
 

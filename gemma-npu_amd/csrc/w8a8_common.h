@@ -238,6 +238,49 @@ __device__ __forceinline__ int8_t quant1_bf16(float v, float s, float rs) {
   return clamp_q(__builtin_rintf(q1));
 }
 
+// Whether a row's scale takes the finite form below: not one of a row with a NaN or an Inf.
+__device__ __forceinline__ bool quant_finite(float s) { return (__float_as_uint(s) & 0x7f800000u) != 0x7f800000u; }
+
+// quant1_bf16 of a value of a row whose scale is finite, as the low byte of the result: |q1| is then at
+// most 127 and a rounding error, so it needs neither the clamp nor the NaN select, and adding 1.5 *
+// 2^23 rounds it to the integer (ties to even, as rint) that stands in the low bits of the sum.  Part
+// of the same self-check.  The row kernels are bound by such instructions: this form takes four and a
+// quarter of a pack per element instead of about ten.
+__device__ __forceinline__ uint32_t quant_bits(float v, float s, float rs) {
+  const float q0 = v * rs;
+  const float r = __builtin_fmaf(-q0, s, v);
+  return __float_as_uint(__builtin_fmaf(r, rs, q0) + 12582912.0f);
+}
+
+// Four int8 codes packed in order.
+__device__ __forceinline__ uint32_t pack_low_bytes(uint32_t a, uint32_t b, uint32_t c, uint32_t d) {
+  return __builtin_amdgcn_perm(b, a, 0x0c0c0400u) | __builtin_amdgcn_perm(d, c, 0x04000c0cu);
+}
+
+// Eight codes of a row with scale s, rs = 1 / s; `finite` = quant_finite(s), the same for the row.
+__device__ __forceinline__ v2u quant8(const float (&v)[8], float s, float rs, bool finite) {
+  v2u w = {0u, 0u};
+  if (finite) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      w[h] = pack_low_bytes(quant_bits(v[4 * h], s, rs), quant_bits(v[4 * h + 1], s, rs),
+                            quant_bits(v[4 * h + 2], s, rs), quant_bits(v[4 * h + 3], s, rs));
+  } else {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) w[i >> 2] |= uint32_t(uint8_t(quant1_bf16(v[i], s, rs))) << (8 * (i & 3));
+  }
+  return w;
+}
+
+// Absmax of packed bf16 pairs: sign-cleared bf16 patterns order as unsigned 16-bit numbers, NaNs above
+// Inf, so one packed maximum serves two elements.  absmax_pair gives the larger half as an fp32.
+typedef unsigned short v2us __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ uint32_t absmax_bf16x2(uint32_t m, uint32_t v) {
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(v2us, m),
+                                                                __builtin_bit_cast(v2us, v & 0x7fff7fffu)));
+}
+__device__ __forceinline__ float absmax_pair(uint32_t m) { return __uint_as_float(max(m & 0xffffu, m >> 16) << 16); }
+
 // ---- XCD-aware block order ---------------------------------------------------------------------
 // Workgroups are dealt to the 8 XCDs round-robin (block b runs on XCD b % 8), each XCD with its
 // own L2.  xcd_remap(b) gives each XCD a contiguous run of logical indices (the last nblocks % 8
