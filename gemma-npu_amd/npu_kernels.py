@@ -55,6 +55,13 @@ def mm_i8(a, b, c, *, wait=True):
     raises instead of truncating to multiples of 512.  With wait=True (the reference's
     contract) c is complete and a is no longer read when this returns.
     """
+    if ops._native is not None and isinstance(b, PackedWeight) and not b.interleave:
+        # device slots: the GEMM and the wait in native code, which declines everything else
+        y = ops._native.gemm_i32(a, -1, 0, b.data, b.N, b.K, c) if c is not None else None
+        if y is not None:
+            if wait and ops._native.wait_stream(c) is None:
+                torch.cuda.current_stream(c.device).synchronize()
+            return c
     if a.dtype != torch.int8 or a.dim() != 2:
         raise TypeError(f"mm_i8: a must be int8 [M, K], got {a.dtype} {tuple(a.shape)}")
     if c.dtype != torch.int32 or c.dim() != 2:

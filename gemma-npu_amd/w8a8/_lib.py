@@ -131,6 +131,16 @@ def lib():
     return _lib
 
 
+def launch_module():
+    """The native launch path (csrc/bind.cpp, w8a8/_launch.so), or None if it is not built or does not
+    fit this torch: the wrappers then make every call through ctypes, with the same results."""
+    try:
+        from . import _launch
+    except ImportError:
+        return None
+    return _launch
+
+
 def call(name, *args):
     """Call `name`; raise W8A8Error with w8a8_last_error() on a non-zero status."""
     L = lib()

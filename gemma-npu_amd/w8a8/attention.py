@@ -22,7 +22,7 @@ import threading
 import torch
 
 from ._lib import call, lib
-from .ops import _stream, current_stream_handle
+from .ops import PackedActivation, _native, _stream, current_stream_handle, packed_act_bytes
 
 _WS = {}
 _WS_LOCK = threading.Lock()
@@ -83,6 +83,10 @@ def attention(q, k, v, q_start=0, window=0, scale=1.0, out=None, return_lse=Fals
     out: optional bf16 [H, Tq, D] destination (any strides with a contiguous last dimension, e.g.
     a transposed view of a [Tq, H, D] tensor).  With return_lse, also the fp32 [H, Tq] natural-log
     logsumexp of the scaled scores (what torch's flash kernels return beside the output)."""
+    if _native is not None and out is None and not return_lse:
+        o = _native.attention(q, k, v, q_start, window, scale, _SPLIT_WS)
+        if o is not None:
+            return o
     _check3(q, "q")
     _check3(k, "k")
     _check3(v, "v")
@@ -119,8 +123,11 @@ def attention_quant(q, k, v, q_start=0, window=0, scale=1.0):
     the quantisation runs in the attention launch itself and the bf16 output is never written; other
     calls (more KV groups, or a plan that merges key parts in a second kernel) run the two steps.
     Bit-identical either way."""
+    if _native is not None:
+        r = _native.attention_quant(q, k, v, q_start, window, scale, _SPLIT_WS)
+        if r is not None:
+            return PackedActivation(r[0], q.shape[1], q.shape[0] * q.shape[2]), r[1]
     from .fused import k_attn_out
-    from .ops import PackedActivation, packed_act_bytes
     _check3(q, "q")
     _check3(k, "k")
     _check3(v, "v")
@@ -173,6 +180,10 @@ def decode(q, k, v, q_pos=None, window=0, scale=1.0, out=None, return_lse=False,
     Returns o [H, D] (into `out` if given), and with return_lse the fp32 [H] logsumexp.
     workspace: a device uint8 tensor of at least decode_workspace_bytes(...) (scratch; nothing is kept
     between calls); by default a buffer cached per device and stream."""
+    if _native is not None and out is None and workspace is None and not return_lse:
+        o = _native.decode(q, k, v, q_pos, window, scale, _WS)
+        if o is not None:
+            return o
     if q.dim() == 3:
         if q.shape[1] != 1:
             raise ValueError(f"decode: expected one query per head, got shape {tuple(q.shape)}")

@@ -1,4 +1,5 @@
-"""Builds libw8a8.so (every HIP source under csrc/) for gfx950 with hipcc.
+"""Builds libw8a8.so (every HIP source under csrc/) for gfx950 with hipcc, and _launch.so (the
+wrappers' launch path, csrc/bind.cpp) with g++.
 
 Run as `python -m w8a8.build` from gemma-npu_amd/, or through __graft_entry__.build().
 Objects go to gemma-npu_amd/_build/, the library next to this file.
@@ -15,6 +16,7 @@ CSRC = os.path.join(ROOT, "csrc")
 INCLUDE = os.path.join(os.path.dirname(ROOT), "include")
 BUILD = os.path.join(ROOT, "_build")
 LIB = os.path.join(PKG, "libw8a8.so")
+LAUNCH = os.path.join(PKG, "_launch.so")
 ARCH = "gfx950"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -38,6 +40,26 @@ def _compile(src):
     return obj
 
 
+def _build_launch():
+    """csrc/bind.cpp (host code against torch's headers) -> w8a8/_launch.so, linked to libw8a8.so."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    rocm = os.path.dirname(os.path.dirname(HIPCC))
+    include = [*cpp_extension.include_paths(), os.path.join(rocm, "include"), sysconfig.get_paths()["include"], INCLUDE]
+    tmp = LAUNCH + ".tmp"
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           *(f"-isystem{d}" for d in include), os.path.join(CSRC, "bind.cpp"), "-o", tmp,
+           f"-L{os.path.join(os.path.dirname(torch.__file__), 'lib')}", "-ltorch_python", "-ltorch", "-ltorch_cpu",
+           "-ltorch_hip", "-lc10", "-lc10_hip", f"-L{os.path.join(rocm, 'lib')}", "-lamdhip64", f"-L{PKG}", "-lw8a8",
+           "-Wl,-rpath,$ORIGIN"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"g++ failed on bind.cpp:\n{r.stdout}\n{r.stderr}")
+    os.replace(tmp, LAUNCH)
+
+
 def build(verbose=False):
     os.makedirs(BUILD, exist_ok=True)
     srcs = sorted(glob.glob(os.path.join(CSRC, "*.hip")))
@@ -49,8 +71,9 @@ def build(verbose=False):
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
     os.replace(tmp, LIB)
+    _build_launch()
     if verbose:
-        print(f"built {LIB} from {len(srcs)} sources", flush=True)
+        print(f"built {LIB} from {len(srcs)} sources and {LAUNCH}", flush=True)
     return LIB
 
 

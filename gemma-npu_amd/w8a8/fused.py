@@ -25,7 +25,7 @@ the tensors' device; there is no CPU fallback.
 import torch
 
 from ._lib import call
-from .ops import PackedActivation, _check, _ld, _same_device, _stream, packed_act_bytes
+from .ops import PackedActivation, _check, _ld, _native, _same_device, _stream, packed_act_bytes
 
 
 def _vec(t, name, n):
@@ -72,6 +72,10 @@ def _rows(t, name, M, N):
 
 def k_in(h, w, eps, packed=False):
     """input_layernorm -> int8 rows for q/k/v: quant(bf16(rms(h, w)))."""
+    if _native is not None and packed:
+        r = _native.k_in(h, w, eps)
+        if r is not None:
+            return PackedActivation(r[0], *h.shape), r[1]
     _check(h, "h", torch.bfloat16)
     M, N = h.shape
     wp = _vec(w, "w", N)
@@ -85,6 +89,10 @@ def k_in(h, w, eps, packed=False):
 def k_qkv(acc, sx, sw, cos, sin, qw, kw, eps, H, KV, D, shared):
     """q/k/v GEMM out -> normed, rotated q [H, T, D], k, v [KV, T, D] (bf16)."""
     H, KV, D = int(H), int(KV), int(D)
+    if _native is not None:
+        r = _native.k_qkv(acc, sx, sw, cos, sin, qw, kw, eps, H, KV, D, bool(shared))
+        if r is not None:
+            return r * 3 if shared else r
     slots = H if shared else H + 2 * KV
     y = _acc(acc, sx, sw, slots * D, dequantised_ok=True)
     T = acc.shape[0]
@@ -164,6 +172,10 @@ def k_attn_out(o, packed=False):
 
 def k_post_attn(acc, sx, sw, res, w_post, w_pre_ff, eps, packed=False):
     """o_proj out -> residual add -> pre-FFN norm -> int8 rows for gate/up: (h, xq, sx)."""
+    if _native is not None and packed:
+        r = _native.k_post_attn(acc, sx, sw, res, w_post, w_pre_ff, eps)
+        if r is not None:
+            return r[0], PackedActivation(r[1], *res.shape), r[2]
     M, N = res.shape
     y = _acc(acc, sx, sw, N, dequantised_ok=True)
     rp, ldr = _rows(res, "res", M, N)
@@ -196,6 +208,10 @@ def k_gelu(acc, sx, sw, I, packed=False):
 
 def k_post_ff(acc, sx, sw, res, w_post_ff, eps, packed=False):
     """down_proj out -> residual add -> int8 rows for the PLE gate: (h, xq, sx)."""
+    if _native is not None and packed:
+        r = _native.k_post_ff(acc, sx, sw, res, w_post_ff, eps)
+        if r is not None:
+            return r[0], PackedActivation(r[1], *res.shape), r[2]
     M, N = res.shape
     y = _acc(acc, sx, sw, N, dequantised_ok=True)
     rp, ldr = _rows(res, "res", M, N)
@@ -215,6 +231,10 @@ def k_post_ff(acc, sx, sw, res, w_post_ff, eps, packed=False):
 
 def k_ple_gate(acc, sx, sw, ple, packed=False):
     """PLE gate out -> gelu * this layer's per-layer input -> int8 rows."""
+    if _native is not None and packed:
+        r = _native.k_ple_gate(acc, sx, sw, ple)
+        if r is not None:
+            return PackedActivation(r[0], *ple.shape), r[1]
     M, N = ple.shape
     y = _acc(acc, sx, sw, N, dequantised_ok=True)
     pp, ldp = _rows(ple, "ple", M, N)
@@ -237,6 +257,10 @@ def k_ple_out(acc, sx, sw, h, w_post_ple, scalar, eps, norm_next=None, packed=Fa
     which is rounded to bf16 first.  With norm_next (the next layer's input-norm weight) the same
     launch also runs that layer's k_in on the rows it writes: returns (out, xq, sx_next), xq packed
     or row-major as k_in's."""
+    if _native is not None and packed and norm_next is not None:
+        r = _native.k_ple_out_k_in(acc, sx, sw, h, w_post_ple, scalar, eps, norm_next)
+        if r is not None:
+            return r[0], PackedActivation(r[1], *h.shape), r[2]
     M, N = h.shape
     y = _acc(acc, sx, sw, N, dequantised_ok=True)
     hp, ldh = _rows(h, "h", M, N)

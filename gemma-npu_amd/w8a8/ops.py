@@ -6,7 +6,11 @@ ready for any later work on the same stream.  There is no CPU fallback.
 """
 import torch
 
-from ._lib import call, lib
+from ._lib import call, launch_module, lib
+
+# The launch path in native code (csrc/bind.cpp), or None where it is not built.  Its functions take the
+# plain case of the wrappers below and return None for everything else, which then runs here.
+_native = launch_module()
 
 EPILOGUES = {"none": 0, "gelu": 1, "residual": 2, "residual_rms": 3}
 
@@ -201,6 +205,10 @@ def pack_act(a, out=None):
 
 def quant_rows_packed(x, out=None, scale=None):
     """Per-row int8 quant of bf16 rows straight into the packed layout -> (PackedActivation, scale)."""
+    if _native is not None and out is None and scale is None:
+        r = _native.quant_packed(x)
+        if r is not None:
+            return PackedActivation(r[0], *x.shape), r[1]
     _check(x, "x", torch.bfloat16)
     M, K = x.shape
     n = packed_act_bytes(M, K)
@@ -221,10 +229,19 @@ def _a_operand(a):
     return a.data_ptr(), _ld(a), 0, a.shape[0], a.shape[1], a
 
 
+def _native_operand(a):
+    """The A operand as the native path takes it: (tensor, M, K), M = -1 for row-major rows."""
+    return (a.data, a.M, a.K) if isinstance(a, PackedActivation) else (a, -1, 0)
+
+
 def gemm_i32(a, w, c=None, tile_cfg=-1, split_k=0):
     """C[M,N] int32 = A[M,K] int8 @ W (exact; npu_kernels.py:40-56).  A is a row-major int8
     tensor or a PackedActivation."""
     w = _packed(w)
+    if _native is not None and tile_cfg == -1 and split_k == 0 and not w.interleave:
+        y = _native.gemm_i32(*_native_operand(a), w.data, w.N, w.K, c)
+        if y is not None:
+            return y if c is None else c
     ap, lda, a_packed, M, K, at = _a_operand(a)
     if K != w.K:
         raise ValueError(f"gemm_i32: A has K={K}, weight has K={w.K}")
@@ -248,6 +265,11 @@ def gemm_bf16(a, sx, w, sw=None, epilogue="none", residual=None, out=None, tile_
     sw = w.sw if sw is None else sw
     if sw is None:
         raise ValueError("gemm_bf16: no per-channel scales")
+    if _native is not None and tile_cfg == -1 and split_k == 0:
+        y = _native.gemm_bf16(*_native_operand(a), sx, w.data, sw, w.N, w.K, w.interleave, EPILOGUES[epilogue],
+                              residual, out)
+        if y is not None:
+            return y if out is None else out
     ap, lda, a_packed, M, K, at = _a_operand(a)
     _check(sx, "sx", torch.float32, 1)
     _check(sw, "sw", torch.float32, 1)
@@ -506,6 +528,10 @@ def linear_bf16(x, w, sw=None, epilogue="none", residual=None, rms_w=None, eps=1
     sw = w.sw if sw is None else sw
     if sw is None:
         raise ValueError("linear_bf16: no per-channel scales")
+    if _native is not None and ws_arg is None:
+        y = _native.linear(x, w.data, sw, w.N, w.K, w.interleave, EPILOGUES[epilogue], residual, rms_w, eps, out)
+        if y is not None:
+            return y if out is None else out
     _check(x, "x", torch.bfloat16)
     _check(sw, "sw", torch.float32, 1)
     M, K = x.shape
@@ -572,6 +598,10 @@ def pack_gemv_weight(w):
 def gemv_bf16(x, w, s, out=None):
     """y = bf16((x @ w^T) * s): torch._weight_int8pack_mm semantics (gemma_npu.py:155-156).
     x bf16 [M<=16, K]; w int8 [N, K] or a GemvWeight; s bf16 or fp32 [N]."""
+    if _native is not None and isinstance(w, GemvWeight):
+        y = _native.gemv(x, w.data, w.N, w.K, s, out)
+        if y is not None:
+            return y if out is None else out
     _check(x, "x", torch.bfloat16)
     packed = isinstance(w, GemvWeight)
     if not packed:

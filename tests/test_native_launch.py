@@ -1,0 +1,124 @@
+"""The native launch path of the torch-facing wrappers (csrc/bind.cpp): what it declines without a GPU,
+and on one that every form a wrapper accepts -- strides, given outputs, row-major and packed operands,
+int32 and bf16 results, stored and missing workspaces -- gives bit for bit what the wrapper's own code
+gives, and that what the wrapper refuses stays refused with the same error."""
+import pytest
+import torch
+
+from w8a8 import _lib, attention, fused, ops
+
+DEV = "cuda"
+
+
+def test_declines_what_it_does_not_take():
+    n = _lib.launch_module()
+    assert n is not None and ops._native is n, "the native launch path is not built"
+    x, w, s = torch.zeros(1, 64, dtype=torch.bfloat16), torch.zeros(64, dtype=torch.int8), torch.zeros(16)
+    assert n.gemv(x, w, 16, 64, s, None) is None          # host tensors
+    assert n.gemv("x", w, 16, 64, s, None) is None        # not a tensor
+    assert n.gemv(x, w, 16) is None                       # another number of arguments
+    assert n.quant_packed(None) is None
+    assert n.quant_packed(torch.nn.Parameter(x)) is None
+    assert n.attention(x, x, x, 0, 0, 1.0, {}) is None
+    assert n.wait_stream(x) is None
+
+
+def both(monkeypatch, call):
+    """call() on the native path and on the wrappers' own code."""
+    outs = []
+    for native in (_lib.launch_module(), None):
+        for m in (ops, fused, attention):
+            monkeypatch.setattr(m, "_native", native)
+        outs.append(call())
+    return outs
+
+
+def flat(r):
+    if isinstance(r, ops.PackedActivation):
+        return [torch.tensor([r.M, r.K]), r.data]
+    if isinstance(r, (tuple, list)):
+        return [t for x in r for t in flat(x)]
+    return [r]
+
+
+def bf(*shape, seed=0):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(torch.bfloat16).to(DEV)
+
+
+def forms():
+    g = torch.Generator().manual_seed(3)
+    w = torch.randint(-127, 128, (96, 128), generator=g, dtype=torch.int8).to(DEV)
+    sw = (torch.rand(96, generator=g) * 0.01).to(DEV)
+    pw, pg, gw = ops.pack_weight(w, "nk", sw=sw), ops.pack_weight(w[:64], "nk", 32, sw=sw[:64]), ops.pack_gemv_weight(w)
+    wide = bf(33, 256, seed=1)
+    x, xs = wide[:, :128].contiguous(), wide[:, 128:]  # xs: rows 256 apart
+    res, one = bf(33, 96, seed=2), bf(1, 128, seed=4)
+    q, sx = ops.quant_rows_packed(x)
+    qr, _ = ops.quant_rows(x)
+    acc = ops.gemm_i32(q, pw)
+    y, n96, sc = ops.gemm_bf16(q, sx, pw), bf(96, seed=5), torch.ones(1, dtype=torch.bfloat16, device=DEV)
+    cs, yq = bf(33, 128, seed=6), bf(33, 4 * 128, seed=7)
+    qa, k, v = bf(2, 40, 128, seed=8), bf(1, 40, 128, seed=9), bf(1, 40, 128, seed=10)
+    qt = bf(40, 2, 128, seed=11).transpose(0, 1)  # [H, T, D] with rows H * D apart
+    return {
+        "gemv": lambda: ops.gemv_bf16(one, gw, sw), "gemv bf16 scales": lambda: ops.gemv_bf16(one, gw, sw.bfloat16()),
+        "gemv strided out": lambda: ops.gemv_bf16(x[:3], gw, sw, torch.zeros(3, 128, dtype=torch.bfloat16, device=DEV)[:, :96]),
+        "linear": lambda: ops.linear_bf16(x, pw), "linear strided": lambda: ops.linear_bf16(xs, pw),
+        "linear empty": lambda: ops.linear_bf16(x[:0], pw),
+        "linear gelu": lambda: ops.linear_bf16(x, pg, epilogue="gelu"),
+        "linear residual": lambda: ops.linear_bf16(x, pw, epilogue="residual", residual=res),
+        "linear residual_rms": lambda: ops.linear_bf16(x, pw, epilogue="residual_rms", residual=res, rms_w=n96),
+        "linear unused residual": lambda: ops.linear_bf16(x, pw, residual=res),
+        "gemm packed": lambda: ops.gemm_i32(q, pw), "gemm rows": lambda: ops.gemm_i32(qr, pw),
+        "gemm given c": lambda: ops.gemm_i32(qr, pw, torch.zeros(33, 100, dtype=torch.int32, device=DEV)[:, :96]),
+        "gemm_bf16": lambda: ops.gemm_bf16(qr, sx, pw, epilogue="residual", residual=res),
+        "quant": lambda: ops.quant_rows_packed(xs), "k_in": lambda: fused.k_in(x, None, 1e-6, packed=True),
+        "k_post_attn": lambda: fused.k_post_attn(y, None, None, res, n96, None, 1e-6, packed=True),
+        "k_post_attn i32": lambda: fused.k_post_attn(acc, sx, sw, res, n96, n96, 1e-6, packed=True),
+        "k_post_ff": lambda: fused.k_post_ff(acc, sx, sw, res, n96, 1e-6, packed=True),
+        "k_ple_gate": lambda: fused.k_ple_gate(y, None, None, res, packed=True),
+        "k_ple_out": lambda: fused.k_ple_out(y, None, None, res, n96, sc, 1e-6, n96, packed=True),
+        "k_ple_out number": lambda: fused.k_ple_out(y, None, None, res, n96, 0.5, 1e-6, n96, packed=True),
+        "k_qkv": lambda: fused.k_qkv(yq, None, None, cs, cs, None, None, 1e-6, 2, 1, 128, False),
+        "k_qkv shared": lambda: fused.k_qkv(yq, None, None, cs, cs, None, None, 1e-6, 4, 0, 128, True),
+        "attention": lambda: attention.attention(qa, k, v), "attention window": lambda: attention.attention(qa, k, v, 0, 16),
+        "attention strided": lambda: attention.attention(qt, k, v, 0, 0, 0.5),
+        "attention_quant": lambda: attention.attention_quant(qa, k, v),
+        "decode": lambda: attention.decode(qa[:, -1], k, v, None, 8), "decode 3-D": lambda: attention.decode(qa[:, -1:], k, v),
+    }
+
+
+@pytest.mark.gpu
+def test_equals_the_wrappers_own_code(monkeypatch):
+    for name, call in forms().items():
+        print(f"native launch path: {name}", flush=True)
+        got, want = (flat(r) for r in both(monkeypatch, call))
+        assert len(got) == len(want), name
+        for a, b in zip(got, want):
+            assert a.shape == b.shape and a.dtype == b.dtype and a.stride() == b.stride(), name
+            if a.dtype == torch.int8 and a.dim() == 1:  # packed rows: the padding of the last block is zero in both
+                assert torch.equal(a, b), name
+            else:
+                assert torch.equal(a.float().nan_to_num(), b.float().nan_to_num()), name
+
+
+@pytest.mark.gpu
+def test_refusals_are_the_wrappers(monkeypatch):
+    w = torch.ones(96, 128, dtype=torch.int8, device=DEV)
+    sw = torch.ones(96, device=DEV)
+    pw, gw, x = ops.pack_weight(w, "nk", sw=sw), ops.pack_gemv_weight(w), bf(2, 128)
+    h = bf(4, 40, 128)
+    calls = [lambda: ops.gemv_bf16(x.float(), gw, sw), lambda: ops.gemv_bf16(x[:, :64], gw, sw),
+             lambda: ops.gemv_bf16(bf(17, 128), gw, sw), lambda: ops.gemv_bf16(x.cpu(), gw, sw),
+             lambda: ops.linear_bf16(bf(128, 2).t(), pw), lambda: ops.linear_bf16(x, pw, epilogue="residual"),
+             lambda: ops.gemm_i32(torch.ones(2, 64, dtype=torch.int8, device=DEV), pw),
+             lambda: fused.k_in(bf(2, 100), None, 1e-6, packed=True),
+             lambda: attention.attention(h, h[:3], h[:3]), lambda: attention.attention(h, h[:1], h[:1], 10),
+             lambda: attention.decode(h[:, 0], h[:1], h[:1], 40)]
+    for i, call in enumerate(calls):
+        def refused():
+            with pytest.raises((TypeError, ValueError, RuntimeError)) as e:
+                call()
+            return e.type, str(e.value)
+        a, b = both(monkeypatch, refused)
+        assert a == b, i
