@@ -586,8 +586,8 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_fwd_kernel(AttnParams p) {
 //
 // Pipeline, one barrier per key block: iteration n computes P V of block n and the S phase and
 // softmax of block n + 1, while the DMAs of K(n + 2) and V(n + 1) are in flight; K, V and P each
-// have two slots (block n in slot n % 2).  Key masking is branch-free so the two phases share one
-// basic block.  The O rescale for a grown row maximum (rare: the reference exponent trails the
+// have two slots (block n in slot n % 2).  Blocks that every row of the tile sees whole are not
+// masked; in the others the key masks are branch-free.  The O rescale for a grown row maximum (rare: the reference exponent trails the
 // maximum lazily) is skipped unless some row of the workgroup grew past a finite maximum.
 //
 // Split tiles park O^T slot-major (slot (dt, rt) of every thread, then the next slot) followed by
@@ -625,7 +625,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_fwd2_kernel(AttnParams p) {
   int* const flag_s = reinterpret_cast<int*>(lds + S::A_OFF + 1024);     // [2][16]
   float* const inv_s = reinterpret_cast<float*>(lds + S::A_OFF + 1152);  // [128]
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int qi = lane & 15, qq = lane >> 4;
 
   // ---- which KV group and query rows (as attn_fwd_kernel) ----------------------------------
@@ -743,6 +743,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_fwd2_kernel(AttnParams p) {
   const int win = p.window;
   const uint32_t wlim = attn_window_limit(win);
   const int Tk = p.Tk;
+  const bool whole_tile = PB * G == 128 && i0 + PB <= Tq;  // no row of the tile is past the queries
 
   // S^T of block n (K slot n % 2), softmax, P rows and rescale factors into slot n % 2
   auto s_phase = [&](int n) __attribute__((always_inline)) {
@@ -772,6 +773,19 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_fwd2_kernel(AttnParams p) {
       for (int j = 0; j < RT; ++j) s[j][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf[i % KR], qf[j][kk], s[j][t], 0, 0, 0);
       if (i + KR < NR) kf[i % KR] = kfrag(i + KR);
     }
+    // every row of the tile sees every key of this block: nothing to mask (the same for the workgroup)
+    const bool inner = whole_tile && kb + BN - 1 <= min(pmin, Tk - 1) && (win <= 0 || kb >= pmax - win + 1);
+    if (!inner) {
+#pragma unroll
+      for (int j = 0; j < RT; ++j)
+#pragma unroll
+        for (int t = 0; t < 2 * NKC; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int key = kb + 32 * (t >> 1) + 8 * qq + 4 * (t & 1) + i;
+            s[j][t][i] = attn_mask(s[j][t][i], valid[j] & attn_key_visible(key, pos[j], Tk, wlim));
+          }
+    }
     bool any = false;
 #pragma unroll
     for (int j = 0; j < RT; ++j) {
@@ -779,11 +793,7 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_fwd2_kernel(AttnParams p) {
 #pragma unroll
       for (int t = 0; t < 2 * NKC; ++t)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const int key = kb + 32 * (t >> 1) + 8 * qq + 4 * (t & 1) + i;
-          s[j][t][i] = attn_mask(s[j][t][i], valid[j] & attn_key_visible(key, pos[j], Tk, wlim));
-          bm = fmaxf(bm, s[j][t][i]);
-        }
+        for (int i = 0; i < 4; ++i) bm = fmaxf(bm, s[j][t][i]);
       bm = lanes4_max(bm);
       const float bmc = bm * c;
       const bool grow = bmc > ms[j] + 8.0f;  // false while every key so far is masked (bmc = -inf)
@@ -863,9 +873,11 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_fwd2_kernel(AttnParams p) {
   };
 
   // ---- main loop --------------------------------------------------------------------------
-  // iteration n: P V of block n and the S phase of block n + 1 (one basic block, so their MFMAs
-  // and LDS reads interleave), with K(n + 2) and V(n + 1) loading into the slots freed by
-  // iteration n - 1
+  // iteration n: the S phase of block n + 1, then P V of block n, with K(n + 2) and V(n + 1) loading
+  // into the slots freed by iteration n - 1.  The S phase first: in the other order the compiler
+  // interleaved the two and, at 256 registers, spilled in the loop and held back LDS reads.  3658
+  // tokens, causal, MI355X: 189.6 us P V first, 172 S first, 166.5 with inner blocks unmasked; half of
+  // the waves in either order spilled and took 182-185, a K ring of 4 / 6 / 8 fragments 169 / 172 / 210.
   if (nblk > 0) {
     if (nblk > 1)
       attn_wait_vmcnt<KU>();  // K(0), V(0) and Q have landed; K(1) may be in flight
@@ -879,8 +891,8 @@ __global__ __launch_bounds__(NW * 64, 1) void attn_fwd2_kernel(AttnParams p) {
     __syncthreads();  // P(n) of every row; K(n + 1) and V(n) in LDS; the other slots free
     if (n + 2 < nblk) issue_k(kb0 + (n + 2) * BN, n & 1);
     issue_v(kb0 + (n + 1) * BN, (n + 1) & 1);
-    pv_phase(n);
     s_phase(n + 1);
+    pv_phase(n);
   }
   if (nblk > 0) {
     attn_wait_vmcnt<0>();
