@@ -1238,53 +1238,45 @@ static bool pipe_tail_is_short(int M, int NP) {
   return tail > 0 && 4 * tail <= cus;
 }
 
-// Tile choice.  Every rule was set by timing the configurations on MI355X (the measured times are
-// tabulated with the design notes); the reasons, briefly:
-//  * One 512-row micro-batch (M <= 1024): the GEMMs are bound by how fast each CU streams its
-//    operands, so small tiles spread over many CUs.  Narrow long-K GEMMs (the output and down
-//    projections) have only ~192 64x64 tiles, one per CU, so four waves split each tile's k-steps
-//    with 512-deep k-tiles (3).  The gate/up GEMM with its GELU epilogue runs on the direct-W 64x256
-//    tile, two blocks per CU (4).  Narrow short-K GEMMs take 64x64 (1).  Wide ones take 64x128 with
-//    two waves per sub-tile while those tiles fit one round on the CUs (2), then one round of
-//    direct-W 64x256 tiles (4), else 64x128 three blocks per CU (0).
-//  * Past one micro-batch: the GELU epilogue on the direct-W 128x256 tile, two blocks per CU (6).
-//    GEMMs up to N = 4096 stream (BM + BN) * K bytes per tile at the per-CU L2 delivery rate, so
-//    one round of the smallest direct-W BMx256 tile that fits the CUs (BM = 96, 128, 160, 192:
-//    7, 5, 8, 9) wins where its bytes per CU undercut the 64x128 three-per-CU tiles'.  The wide
-//    int32 GEMMs (N >= 8192) take the software-pipelined persistent 256x256 kernel (10), which
-//    reads each weight half as often, unless its last round would be nearly empty; everything
-//    else the 128x256 two-per-CU tile (6), or 64x128 (0) where 6's tiles are fewer than the CUs or
-//    leave a nearly empty last round.
+// Tile choice, set by timing every configuration on MI355X over 18 (N, K, epilogue) of the E2B layers at
+// 20 row counts from 1 to 8192 (us below: the configuration named against the next best or the
+// general one).  A tile's time is the stream of its (BM + BN) * K bytes into its CU, about 30 bytes per
+// clock, so while a configuration's tiles fit one round on the CUs the smallest such tile wins, and a
+// nearly empty second round costs a whole one:
+//  * 64x64, four waves splitting each k-tile's steps (3): every launch whose 64x64 tiles fit, long K or
+//    short (qkv 1536 x 2560: 6.0 at M = 77 against 8.2 on 64x128; 1536 x 256 at M = 3658: 6.4 against
+//    8.1-8.7).  K below 512 is one of its k-tiles, without a ring to fill: two waves per 64x64 tile (1),
+//    then 64x256 (4; 256 x 1536 at M = 3658: 6.9 against 8.1) or, where int32 results make the store
+//    the larger part, 64x128 (0).
+//  * 64x128 with two waves per sub-tile (2) where those fit: for long K (6144 x 1536 at M = 1100: 24.9
+//    against 28.9 on 64x256, and 44.1 on 128x256), for int32 results, whose 64x256 tile has twice the
+//    store behind its last k-step (6144 at M = 256: 8.9 against 9.8), and for few rows.
+//  * the direct-W BMx256 tiles, smallest BM whose tiles fit: 64 (4), 96 (7), 128 (6, two blocks per CU;
+//    5, W further ahead, for long K), 160 (8), 192 (9): 5120 x 1536 at M = 1100: 14.1 on 96 against 17.4.
+//    The two largest only where they fill most of the CUs (24576 with GELU at M = 300: 20.9 on 192 of
+//    them, 19.1 on 480 64x256 tiles), and not 192 with GELU, whose epilogue is then long and alone on its
+//    CU (12288 at M = 900: 25.3 against 24.7).
+//  * more than one round: 64x256 up to 1024 rows (gate/up with GELU, M = 512: 16.2); past that 128x256,
+//    two blocks per CU (6), whose second block multiplies while the first stores; 96x256 (7) instead
+//    where 6's last round would be nearly empty (6144 at M = 2900: 35.0 against 39.1).  Wide int32 GEMMs
+//    take the software-pipelined persistent 256x256 kernel (10), which reads each weight half as
+//    often, unless its last round would be nearly empty.
 int gemm_pick_config(int M, int NP, int K, int epi) {
   const int cus = cu_count();
-  if (M <= 1024) {
-    if (K >= 2048 && NP <= 4096) return CFG_64x64_KW4;
-    if (epi == EPI_GELU) return CFG_DW_64x256;
-    if (NP <= 2048) return CFG_64x64;
-    const int mt = (M + 63) / 64;
-    if (mt * ((NP + 127) / 128) <= cus) return CFG_64x128_KW2;
-    return mt * ((NP + 255) / 256) <= cus ? CFG_DW_64x256 : CFG_64x128;
-  }
-  if (epi == EPI_GELU) return CFG_DW_128x256;
-  auto tiles = [&](int bm, int bn) { return ((M + bm - 1) / bm) * ((NP + bn - 1) / bn); };
-  if (K >= 1024 && NP <= 4096) {
-    // one round of direct-W BMx256 tiles, smallest BM first, where the busiest CU moves fewer bytes
-    // than on the 64x128 three-per-CU tiles
-    const int cost0 = (tiles(64, 128) + cus - 1) / cus * (64 + 128);
-    constexpr int kBm[4] = {96, 128, 160, 192};
-    constexpr int kCfgOf[4] = {CFG_DW_96x256, CFG_DW_128x256_PW8, CFG_DW_160x256, CFG_DW_192x256};
-    for (int i = 0; i < 4; ++i)
-      if (tiles(kBm[i], 256) <= cus) {
-        if (kBm[i] + 256 < cost0) return kCfgOf[i];
-        break;
-      }
-  }
-  const bool pipe = NP >= 8192 && epi == EPI_I32 && !pipe_tail_is_short(M, NP);
-  if (M > 8192) return pipe ? CFG_PIPE_256x256 : CFG_DW_128x256;
-  if (K >= 4096 && NP <= 2048) return CFG_DW_128x256;  // long-K narrow past one round of 128x256
-  if (NP >= 8192) return pipe ? CFG_PIPE_256x256 : CFG_DW_128x256;
-  const int t6 = tiles(128, 256), tail = t6 % cus;
-  return t6 >= cus && !(tail > 0 && 4 * tail <= cus) ? CFG_DW_128x256 : CFG_64x128;
+  auto fit = [&](int bm, int bn) { return int64_t((M + bm - 1) / bm) * ((NP + bn - 1) / bn) <= cus; };
+  if (K < 512) return fit(64, 64) ? CFG_64x64 : epi == EPI_I32 ? CFG_64x128 : CFG_DW_64x256;
+  if (fit(64, 64)) return CFG_64x64_KW4;
+  if (fit(64, 128) && (K >= 2048 || epi == EPI_I32 || M <= 256)) return CFG_64x128_KW2;
+  if (fit(64, 256)) return CFG_DW_64x256;
+  if (fit(96, 256)) return CFG_DW_96x256;
+  if (fit(128, 256)) return epi == EPI_GELU || K < 2048 ? CFG_DW_128x256 : CFG_DW_128x256_PW8;
+  auto full = [&](int bm) { return 20 * int64_t((M + bm - 1) / bm) * ((NP + 255) / 256) >= 17 * cus; };
+  if (fit(160, 256) && full(160)) return CFG_DW_160x256;
+  if (fit(192, 256) && full(192) && epi != EPI_GELU) return CFG_DW_192x256;
+  if (M <= 1024) return CFG_DW_64x256;
+  if (NP >= 8192 && epi == EPI_I32 && !pipe_tail_is_short(M, NP)) return CFG_PIPE_256x256;
+  const int tail = ((M + 127) / 128) * ((NP + 255) / 256) % cus;
+  return M <= 8192 && NP < 8192 && tail > 0 && 4 * tail <= cus ? CFG_DW_96x256 : CFG_DW_128x256;
 }
 
 int gemm_launch(const GemmParams& p, int epi, int cfg, bool a_packed, hipStream_t stream) {

@@ -45,3 +45,26 @@ def test_auto_tile_int32_and_dequant_exact(M, N, K):
     r = torch.randn(M, N, generator=g, device=DEV).to(torch.bfloat16)
     yr = ops.gemm_bf16(a, sx, pw, epilogue="residual", residual=r)
     assert torch.equal(yr.view(torch.int16), (ref + r).view(torch.int16)), f"residual mismatch at M={M} N={N} K={K}"
+
+
+# Launches whose tiles of one size just fill the 256 CUs, and one tile more: 64x64, 64x128, and the
+# BMx256 tiles (also at the share of the CUs the two largest must fill), short K, GELU pairs.
+EDGES = [(64, 16384, 512), (64, 16400, 512), (4096, 256, 576), (4097, 256, 576), (128, 8208, 2048), (1024, 2048, 2048),
+         (1025, 2048, 1536), (96, 16400, 512), (1536, 4096, 512), (1537, 4096, 512), (2100, 4096, 512),
+         (2560, 3600, 512), (1280, 4400, 512), (3072, 4096, 512), (4096, 256, 448), (4097, 256, 448), (300, 24576, 512)]
+
+
+@pytest.mark.parametrize("M,N,K", EDGES)
+def test_auto_tile_exact_at_the_one_round_edges(M, N, K):
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    a = torch.randint(-128, 128, (M, K), generator=g, dtype=torch.int8, device=DEV)
+    w = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8, device=DEV)
+    sx, sw = torch.rand(M, generator=g, device=DEV) * 0.05, torch.rand(N, generator=g, device=DEV) * 0.01
+    print(f"one-round edge M={M} N={N} K={K}", flush=True)
+    want = (a.double() @ w.double().T).int()
+    assert torch.equal(ops.gemm_i32(a, ops.pack_weight(w, "nk")), want)
+    y = ((want.float() * sx[:, None]) * sw[None, :]).to(torch.bfloat16)
+    assert torch.equal(ops.gemm_bf16(a, sx, ops.pack_weight(w, "nk", sw=sw)), y)
+    if N % 64 == 0:
+        got = ops.gemm_bf16(a, sx, ops.pack_weight(w, "nk", N // 2, sw=sw), epilogue="gelu")
+        assert torch.equal(got, ops.gelu_mul_bf16(y))
