@@ -233,18 +233,15 @@ struct RowIn {
   }
 };
 
-// Widen 8 signed bytes (two dwords) to 8 bf16 values, exactly.
+// Widen 8 signed bytes (two dwords) to 8 bf16 values, exactly: a sign-extending conversion per byte and
+// one packed conversion (nothing to round: |w| <= 128) per pair.
 __device__ __forceinline__ v8bf widen8(uint32_t lo, uint32_t hi) {
   v4u r;
 #pragma unroll
   for (int i = 0; i < 2; ++i) {
     const uint32_t d = i ? hi : lo;
-    const float f0 = float(int8_t(d & 0xff));
-    const float f1 = float(int8_t((d >> 8) & 0xff));
-    const float f2 = float(int8_t((d >> 16) & 0xff));
-    const float f3 = float(int8_t(d >> 24));
-    r[2 * i] = (__float_as_uint(f0) >> 16) | (__float_as_uint(f1) & 0xffff0000u);
-    r[2 * i + 1] = (__float_as_uint(f2) >> 16) | (__float_as_uint(f3) & 0xffff0000u);
+    r[2 * i] = pack_bf16x2(float(int8_t(d & 0xff)), float(int8_t((d >> 8) & 0xff)));
+    r[2 * i + 1] = pack_bf16x2(float(int8_t((d >> 16) & 0xff)), float(int8_t(d >> 24)));
   }
   return __builtin_bit_cast(v8bf, r);
 }
@@ -457,7 +454,7 @@ __global__ __launch_bounds__(NWB * 64) void gemv_kernel(GemvParams p) {
 //    made in LDS (PRO 3: the residual stream's norm, a row of 3 * 512; 4: the attention merge; 5:
 //    copied from x);
 //  * the tiles are dealt in units, `gpb` groups of `split` waves to a workgroup (gemv1_plan), and a
-//    wave multiplies no fragment past K: widening a KiB of bytes takes a SIMD about 130 clocks.
+//    wave multiplies no fragment past K: widening a KiB of bytes takes a SIMD about 100 clocks.
 // For the same reason a weight with few tiles (N = 1536: 96 of 16 rows on 256 CUs) is dealt in halves
 // (wide down 12288 x 1536: 9.6 us in whole tiles, 7.0 in halves): with HALF a unit is 8 weight rows, and a fragment load takes them from two
 // k-blocks at once: lane l holds row l % 8 of the unit, of k-block 2 q + (l % 16 >= 8) for pair q,
@@ -475,7 +472,7 @@ __global__ __launch_bounds__(PRO == 4 ? 1024 : 768) void gemv1_kernel(GemvParams
   constexpr bool SPLIT_ROWS = HALF || ACT == 1;    // a unit is 8 output columns
   constexpr bool PAIR = ACT == 1 && !HALF;         // gate and up rows in one fragment
   __shared__ v4f red[16][TPW][4];                  // per wave: rows 4j .. 4j+3 of its tile
-  __shared__ __attribute__((aligned(16))) uint16_t xs[XS];                    // the row
+  __shared__ __attribute__((aligned(16))) uint16_t xs[XS + 16];               // the row, and a piece of zeros
   __shared__ __attribute__((aligned(16))) uint16_t hs[NORM ? PRO * 512 : 8];  // NORM: the first norm's row
   __shared__ float mw[PRO == 4 ? MERGE_HEADS * (DEC_MERGE_IN_GEMV_CHUNKS + 1) : 1];  // PRO 4: chunk weights
   const int lane = threadIdx.x & 63;
@@ -520,19 +517,21 @@ __global__ __launch_bounds__(PRO == 4 ? 1024 : 768) void gemv1_kernel(GemvParams
     for (int t = 0; t < TPW; ++t) w[t] = load_weight<PACKED>(rw, ok ? wbase[t] + uint32_t(kb) * W_KB : PAST);
   };
 
+  const int row_end = (HALF ? (p.KB + 1) & ~1 : p.KB) * 64;  // the row's elements that are read
+  if (threadIdx.x < 2) *reinterpret_cast<v4i*>(xs + XS + 8 * threadIdx.x) = v4i{0, 0, 0, 0};
   v4i wv[U][TPW];
   if constexpr (PRO == 5) {
     // The row's pieces of 8 are asked for before the weights, two per thread (all of it from 12 waves
     // on); a wait inside a loop would be one for the weights too.
     const int k0 = int(threadIdx.x) * 8, nt8 = int(blockDim.x) * 8, k1 = k0 + nt8;
-    for (int k = k1 + nt8; k < p.KB * 64; k += nt8)
+    for (int k = k1 + nt8; k < row_end; k += nt8)
       *reinterpret_cast<v4i*>(xs + k) = buf_load16(rx, k < p.K ? uint32_t(k) * 2u : PAST);
     const v4i x0 = buf_load16(rx, k0 < p.K ? uint32_t(k0) * 2u : PAST);
     const v4i x1 = buf_load16(rx, k1 < p.K ? uint32_t(k1) * 2u : PAST);
 #pragma unroll
     for (int u = 0; u < U; ++u) load_w(ks + u * split, wv[u]);
-    if (k0 < p.KB * 64) *reinterpret_cast<v4i*>(xs + k0) = x0;
-    if (k1 < p.KB * 64) *reinterpret_cast<v4i*>(xs + k1) = x1;
+    if (k0 < row_end) *reinterpret_cast<v4i*>(xs + k0) = x0;
+    if (k1 < row_end) *reinterpret_cast<v4i*>(xs + k1) = x1;
   } else {
 #pragma unroll
     for (int u = 0; u < U; ++u) load_w(ks + u * split, wv[u]);
@@ -543,6 +542,13 @@ __global__ __launch_bounds__(PRO == 4 ? 1024 : 768) void gemv1_kernel(GemvParams
   }
   __syncthreads();
 
+  // This lane's piece of the row for step st: activation column 0 takes it (with HALF column 0 the even
+  // k-blocks and column 1 the odd ones), the others read a piece of zeros, so that the reads take no
+  // branch and stand ahead of the MFMAs.  The row is zero from K up to the next k-block (with HALF, the
+  // next pair).
+  const bool column = i < (HALF ? 2 : 1);
+  const uint16_t* const xbase = column ? xs + (HALF ? i * 64 : 0) + j * 16 : xs + XS;
+  const int xstep = column ? (HALF ? 128 : 64) : 0;
   v4f acc[TPW];
 #pragma unroll
   for (int t = 0; t < TPW; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
@@ -553,16 +559,10 @@ __global__ __launch_bounds__(PRO == 4 ? 1024 : 768) void gemv1_kernel(GemvParams
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      // activation column i: with HALF column 0 takes the even k-block, column 1 the odd one
       const int st = st0 + u * split;
       if (st >= nstep) break;
-      const int kb = HALF ? 2 * st + i : st;
-      v4i xa = {0, 0, 0, 0}, xb = {0, 0, 0, 0};
-      if (i < (HALF ? 2 : 1) && kb < p.KB && kb * 64 + j * 16 < p.K) {
-        const v4i* xv = reinterpret_cast<const v4i*>(xs + kb * 64 + j * 16);
-        xa = xv[0];
-        xb = xv[1];
-      }
+      const uint16_t* xv = xbase + st * xstep;
+      const v4i xa = *reinterpret_cast<const v4i*>(xv), xb = *reinterpret_cast<const v4i*>(xv + 8);
 #pragma unroll
       for (int t = 0; t < TPW; ++t) acc[t] = mma_block(wv[u][t], xa, xb, acc[t]);
     }
@@ -686,10 +686,11 @@ static bool gemv1_takes(const GemvParams& p) {
 // U fragments in flight per wave: all of a wave's share in one round where the registers allow it.
 // MI355X, weights cold, a chain of launches replayed from a graph (a chain of empty ones takes 1.9 us
 // each), us per launch, before (one tile per workgroup of 8 or 16 waves, the row made by one wave, the
-// scales fetched after the sums) -> now: o 2048 x 1536 4.5 -> 3.6, 4096 x 1536 5.5 -> 4.2; qkv 1536 x
-// 2560 with its norm 6.3 -> 4.8; gate/up with norm and GELU 1536 x 12288 10.6 -> 7.7, x 24576 13.8 ->
-// 12.1; down 6144 x 1536 7.0 -> 5.0, 12288 x 1536 10.5 -> 7.0; per-layer gate 1536 x 256 with norm
-// 6.3 -> 4.6, projection 256 x 1536 3.3 -> 3.0.
+// scales fetched after the sums) -> now: o 2048 x 1536 4.5 -> 3.4, 4096 x 1536 5.5 -> 4.2; qkv 1536 x
+// 2560 with its norm 6.3 -> 4.6; gate/up with norm and GELU 1536 x 12288 10.6 -> 7.0, x 24576 13.8 ->
+// 10.9; down 6144 x 1536 7.0 -> 4.9, 12288 x 1536 10.5 -> 7.0; per-layer gate 1536 x 256 with norm
+// 6.3 -> 4.5, projection 256 x 1536 3.3 -> 3.0.  (4.8, 7.7, 12.1 for the qkv and gate/up rows before the
+// packed widening and the branch-free row reads.)
 template <bool PACKED, int ACT, int PRO>
 static void gemv1_launch(const GemvParams& p0, hipStream_t stream) {
   GemvParams p = p0;
