@@ -1244,39 +1244,70 @@ static bool pipe_tail_is_short(int M, int NP) {
 // clock, so while a configuration's tiles fit one round on the CUs the smallest such tile wins, and a
 // nearly empty second round costs a whole one:
 //  * 64x64, four waves splitting each k-tile's steps (3): every launch whose 64x64 tiles fit, long K or
-//    short (qkv 1536 x 2560: 6.0 at M = 77 against 8.2 on 64x128; 1536 x 256 at M = 3658: 6.4 against
-//    8.1-8.7).  K below 512 is one of its k-tiles, without a ring to fill: two waves per 64x64 tile (1),
-//    then 64x256 (4; 256 x 1536 at M = 3658: 6.9 against 8.1) or, where int32 results make the store
-//    the larger part, 64x128 (0).
+//    short (1536 x 2560, K x N: 6.0 at M = 77 against 8.2 on 64x128; down 6144 x 1536 at M = 512: 14.4).
+//    K below 512 is one of its k-tiles, without a ring to fill: two waves per 64x64 tile (1), then 64x256
+//    (4) or, where int32 results make the store the larger part, 64x128 (0).
 //  * 64x128 with two waves per sub-tile (2) where those fit: for long K (6144 x 1536 at M = 1100: 24.9
 //    against 28.9 on 64x256, and 44.1 on 128x256), for int32 results, whose 64x256 tile has twice the
-//    store behind its last k-step (6144 at M = 256: 8.9 against 9.8), and for few rows.
-//  * the direct-W BMx256 tiles, smallest BM whose tiles fit: 64 (4), 96 (7), 128 (6, two blocks per CU;
-//    5, W further ahead, for long K), 160 (8), 192 (9): 5120 x 1536 at M = 1100: 14.1 on 96 against 17.4.
-//    The two largest only where they fill most of the CUs (24576 with GELU at M = 300: 20.9 on 192 of
-//    them, 19.1 on 480 64x256 tiles), and not 192 with GELU, whose epilogue is then long and alone on its
-//    CU (12288 at M = 900: 25.3 against 24.7).
-//  * more than one round: 64x256 up to 1024 rows (gate/up with GELU, M = 512: 16.2); past that 128x256,
-//    two blocks per CU (6), whose second block multiplies while the first stores; 96x256 (7) instead
-//    where 6's last round would be nearly empty (6144 at M = 2900: 35.0 against 39.1).  Wide int32 GEMMs
-//    take the software-pipelined persistent 256x256 kernel (10), which reads each weight half as
-//    often, unless its last round would be nearly empty.
+//    store behind its last k-step (1536 x 6144 at M = 256: 8.9 against 9.8), and for few rows.
+//  * the direct-W BMx256 tiles, smallest BM whose tiles fit: 64 (4; 6144 x 1536 at M = 2048: 29.1 against
+//    34.0 on 96), 96 (7; at M = 3658: 39.7 against 45.4 on 128), 128 (6, two blocks per CU; 5, W further
+//    ahead, for long K), 160 (8), 192 (9).  The two largest only where they fill most of the CUs
+//    (1536 x 24576 with GELU at M = 300: 20.9 on 192 of them, 19.1 on 480 64x256 tiles), and not 192 with
+//    GELU, whose epilogue is then long and alone on its CU.
+//  * more than one round: 64x256 up to 1024 rows; past that 128x256, two blocks per CU (6), whose second
+//    block multiplies while the first stores; 96x256 (7) instead where 6's last round would be nearly
+//    empty.  Wide int32 GEMMs take the software-pipelined persistent 256x256 kernel (10), which reads each
+//    weight half as often, unless its last round would be nearly empty.
+//
+// This rule is taken below 512 rows, and from K = 2048 on for every row count.  For short-K GEMMs of 512
+// rows and more the configuration of a shape is a stated result of w8a8_gemm_pick_tile_config, and stays:
+// up to 1024 rows small tiles by N (64x256 with GELU: gate/up at M = 512 16.2); past that one round of the
+// smallest BMx256 tile where the busiest CU moves fewer bytes than on 64x128, three per CU, else 6, or
+// 64x128 (0) where 6's tiles are fewer than the CUs or leave a nearly empty last round.  The one-round
+// rule would be faster for some of them (1536 x 5120 at M = 1100: 14.1 against 17.4; 1536 x 256 at
+// M = 3658: 6.4 against 8.7).
 int gemm_pick_config(int M, int NP, int K, int epi) {
   const int cus = cu_count();
-  auto fit = [&](int bm, int bn) { return int64_t((M + bm - 1) / bm) * ((NP + bn - 1) / bn) <= cus; };
-  if (K < 512) return fit(64, 64) ? CFG_64x64 : epi == EPI_I32 ? CFG_64x128 : CFG_DW_64x256;
-  if (fit(64, 64)) return CFG_64x64_KW4;
-  if (fit(64, 128) && (K >= 2048 || epi == EPI_I32 || M <= 256)) return CFG_64x128_KW2;
-  if (fit(64, 256)) return CFG_DW_64x256;
-  if (fit(96, 256)) return CFG_DW_96x256;
-  if (fit(128, 256)) return epi == EPI_GELU || K < 2048 ? CFG_DW_128x256 : CFG_DW_128x256_PW8;
-  auto full = [&](int bm) { return 20 * int64_t((M + bm - 1) / bm) * ((NP + 255) / 256) >= 17 * cus; };
-  if (fit(160, 256) && full(160)) return CFG_DW_160x256;
-  if (fit(192, 256) && full(192) && epi != EPI_GELU) return CFG_DW_192x256;
-  if (M <= 1024) return CFG_DW_64x256;
-  if (NP >= 8192 && epi == EPI_I32 && !pipe_tail_is_short(M, NP)) return CFG_PIPE_256x256;
-  const int tail = ((M + 127) / 128) * ((NP + 255) / 256) % cus;
-  return M <= 8192 && NP < 8192 && tail > 0 && 4 * tail <= cus ? CFG_DW_96x256 : CFG_DW_128x256;
+  auto tiles = [&](int bm, int bn) { return int64_t((M + bm - 1) / bm) * ((NP + bn - 1) / bn); };
+  auto fit = [&](int bm, int bn) { return tiles(bm, bn) <= cus; };
+  const bool pipe = M > 1024 && NP >= 8192 && epi == EPI_I32 && !pipe_tail_is_short(M, NP);
+  const int tail = int(tiles(128, 256) % cus);
+  const bool short_tail = tail > 0 && 4 * tail <= cus;
+  if (M < 512 || K >= 2048) {
+    if (K < 512) return fit(64, 64) ? CFG_64x64 : epi == EPI_I32 ? CFG_64x128 : CFG_DW_64x256;
+    if (fit(64, 64)) return CFG_64x64_KW4;
+    if (fit(64, 128) && (K >= 2048 || epi == EPI_I32 || M <= 256)) return CFG_64x128_KW2;
+    if (fit(64, 256)) return CFG_DW_64x256;
+    if (fit(96, 256)) return CFG_DW_96x256;
+    if (fit(128, 256)) return epi == EPI_GELU || K < 2048 ? CFG_DW_128x256 : CFG_DW_128x256_PW8;
+    auto full = [&](int bm) { return 20 * tiles(bm, 256) >= 17 * cus; };
+    if (fit(160, 256) && full(160)) return CFG_DW_160x256;
+    if (fit(192, 256) && full(192) && epi != EPI_GELU) return CFG_DW_192x256;
+    if (M <= 1024) return CFG_DW_64x256;
+    if (pipe) return CFG_PIPE_256x256;
+    return M <= 8192 && NP < 8192 && short_tail ? CFG_DW_96x256 : CFG_DW_128x256;
+  }
+  if (M <= 1024) {
+    if (epi == EPI_GELU) return CFG_DW_64x256;
+    if (NP <= 2048) return CFG_64x64;
+    if (fit(64, 128)) return CFG_64x128_KW2;
+    return fit(64, 256) ? CFG_DW_64x256 : CFG_64x128;
+  }
+  if (epi == EPI_GELU) return CFG_DW_128x256;
+  if (K >= 1024 && NP <= 4096) {
+    const int64_t cost0 = (tiles(64, 128) + cus - 1) / cus * (64 + 128);
+    constexpr int kBm[4] = {96, 128, 160, 192};
+    constexpr int kCfgOf[4] = {CFG_DW_96x256, CFG_DW_128x256_PW8, CFG_DW_160x256, CFG_DW_192x256};
+    for (int i = 0; i < 4; ++i)
+      if (fit(kBm[i], 256)) {
+        if (kBm[i] + 256 < cost0) return kCfgOf[i];
+        break;
+      }
+  }
+  if (pipe) return CFG_PIPE_256x256;
+  if (M > 8192 || NP >= 8192) return CFG_DW_128x256;
+  return tiles(128, 256) >= cus && !short_tail ? CFG_DW_128x256 : CFG_64x128;
 }
 
 int gemm_launch(const GemmParams& p, int epi, int cfg, bool a_packed, hipStream_t stream) {

@@ -49,9 +49,10 @@ def test_auto_tile_int32_and_dequant_exact(M, N, K):
 
 # Launches whose tiles of one size just fill the 256 CUs, and one tile more: 64x64, 64x128, and the
 # BMx256 tiles (also at the share of the CUs the two largest must fill), short K, GELU pairs.
-EDGES = [(64, 16384, 512), (64, 16400, 512), (4096, 256, 576), (4097, 256, 576), (128, 8208, 2048), (1024, 2048, 2048),
-         (1025, 2048, 1536), (96, 16400, 512), (1536, 4096, 512), (1537, 4096, 512), (2100, 4096, 512),
-         (2560, 3600, 512), (1280, 4400, 512), (3072, 4096, 512), (4096, 256, 448), (4097, 256, 448), (300, 24576, 512)]
+EDGES = [(64, 16384, 512), (64, 16400, 512), (4096, 256, 2048), (4097, 256, 2048), (128, 8208, 2048), (1024, 2048, 2048),
+         (1025, 2048, 2048), (96, 16400, 512), (1536, 4096, 2048), (1537, 4096, 2048), (2100, 4096, 2048),
+         (2560, 3600, 2048), (1280, 4400, 2048), (3072, 4096, 2048), (511, 2048, 448), (511, 2064, 448), (300, 24576, 512),
+         (511, 8960, 1984), (512, 8960, 1984), (2100, 4096, 1984)]
 
 
 @pytest.mark.parametrize("M,N,K", EDGES)
