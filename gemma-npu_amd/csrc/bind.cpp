@@ -144,7 +144,7 @@ PyObject* gemv(PyObject* const* a) {
   return wrap(y);
 }
 
-// x, w.data, sw, N, K, interleave, epilogue, residual, rms_w, eps, out
+// x, w.data, sw, N, K, interleave, epilogue, residual, rms_w, eps, out, workspace
 PyObject* linear(PyObject* const* a) {
   Call c;
   const Tensor& x = c.rows(a[0], at::kBFloat16);
@@ -166,8 +166,9 @@ PyObject* linear(PyObject* const* a) {
   if (a[8] != Py_None) rw = bf(c.vec(a[8], at::kBFloat16));
   const float eps = real(a[9]);
   const Tensor y = output(c, a[10], M, epi == 1 ? I : N, at::kBFloat16);
-  const int64_t bytes = w8a8_linear_workspace_bytes(M, N, K);
-  const Tensor ws = c.make({std::max<int64_t>(bytes, 256)}, at::kByte);
+  // the C entry checks a given workspace's size
+  const Tensor ws = a[11] != Py_None ? c.vec(a[11], at::kByte)
+                                     : c.make({std::max<int64_t>(w8a8_linear_workspace_bytes(M, N, K), 256)}, at::kByte);
   const hipStream_t st = c.stream();
   launch([&] {
     return w8a8_linear_bf16(bf(x), ld(x), i8(w), f32(sw), M, N, K, int(epi), I, res, ldr, rw, eps, bfo(y), ld(y),
@@ -517,7 +518,7 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 #define W8A8_ENTRY(name, n) \
   {#name, reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(&entry<name, n>)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
-    W8A8_ENTRY(gemv, 6),        W8A8_ENTRY(linear, 11),         W8A8_ENTRY(gemm_i32, 7),  W8A8_ENTRY(gemm_bf16, 12),
+    W8A8_ENTRY(gemv, 6),        W8A8_ENTRY(linear, 12),         W8A8_ENTRY(gemm_i32, 7),  W8A8_ENTRY(gemm_bf16, 12),
     W8A8_ENTRY(quant_packed, 1), W8A8_ENTRY(k_in, 3),           W8A8_ENTRY(k_post_attn, 7), W8A8_ENTRY(k_post_ff, 6),
     W8A8_ENTRY(k_ple_gate, 4),  W8A8_ENTRY(k_ple_out_k_in, 8),  W8A8_ENTRY(k_qkv, 12),    W8A8_ENTRY(attention, 7),
     W8A8_ENTRY(attention_quant, 7), W8A8_ENTRY(decode, 7),      W8A8_ENTRY(wait_stream, 1),

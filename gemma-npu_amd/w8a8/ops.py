@@ -528,8 +528,8 @@ def linear_bf16(x, w, sw=None, epilogue="none", residual=None, rms_w=None, eps=1
     sw = w.sw if sw is None else sw
     if sw is None:
         raise ValueError("linear_bf16: no per-channel scales")
-    if _native is not None and ws_arg is None:
-        y = _native.linear(x, w.data, sw, w.N, w.K, w.interleave, EPILOGUES[epilogue], residual, rms_w, eps, out)
+    if _native is not None:
+        y = _native.linear(x, w.data, sw, w.N, w.K, w.interleave, EPILOGUES[epilogue], residual, rms_w, eps, out, ws_arg)
         if y is not None:
             return y if out is None else out
     _check(x, "x", torch.bfloat16)

@@ -52,6 +52,7 @@ def forms():
     pw, pg, gw = ops.pack_weight(w, "nk", sw=sw), ops.pack_weight(w[:64], "nk", 32, sw=sw[:64]), ops.pack_gemv_weight(w)
     wide = bf(33, 256, seed=1)
     x, xs = wide[:, :128].contiguous(), wide[:, 128:]  # xs: rows 256 apart
+    ws = ops.workspace(x.device, ops.linear_workspace_bytes(33, 96, 128))
     res, one = bf(33, 96, seed=2), bf(1, 128, seed=4)
     q, sx = ops.quant_rows_packed(x)
     qr, _ = ops.quant_rows(x)
@@ -65,6 +66,7 @@ def forms():
         "gemv strided out": lambda: ops.gemv_bf16(x[:3], gw, sw, torch.zeros(3, 128, dtype=torch.bfloat16, device=DEV)[:, :96]),
         "linear": lambda: ops.linear_bf16(x, pw), "linear strided": lambda: ops.linear_bf16(xs, pw),
         "linear empty": lambda: ops.linear_bf16(x[:0], pw),
+        "linear given workspace": lambda: ops.linear_bf16(x, pw, ws_arg=ws),
         "linear gelu": lambda: ops.linear_bf16(x, pg, epilogue="gelu"),
         "linear residual": lambda: ops.linear_bf16(x, pw, epilogue="residual", residual=res),
         "linear residual_rms": lambda: ops.linear_bf16(x, pw, epilogue="residual_rms", residual=res, rms_w=n96),
@@ -108,7 +110,9 @@ def test_refusals_are_the_wrappers(monkeypatch):
     sw = torch.ones(96, device=DEV)
     pw, gw, x = ops.pack_weight(w, "nk", sw=sw), ops.pack_gemv_weight(w), bf(2, 128)
     h = bf(4, 40, 128)
+    small = torch.empty(8, dtype=torch.uint8, device=DEV)
     calls = [lambda: ops.gemv_bf16(x.float(), gw, sw), lambda: ops.gemv_bf16(x[:, :64], gw, sw),
+             lambda: ops.linear_bf16(x, pw, ws_arg=small),
              lambda: ops.gemv_bf16(bf(17, 128), gw, sw), lambda: ops.gemv_bf16(x.cpu(), gw, sw),
              lambda: ops.linear_bf16(bf(128, 2).t(), pw), lambda: ops.linear_bf16(x, pw, epilogue="residual"),
              lambda: ops.gemm_i32(torch.ones(2, 64, dtype=torch.int8, device=DEV), pw),
