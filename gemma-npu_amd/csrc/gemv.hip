@@ -456,22 +456,26 @@ __global__ __launch_bounds__(NWB * 64) void gemv_kernel(GemvParams p) {
 //  * the tiles are dealt in units, `gpb` groups of `split` waves to a workgroup (gemv1_plan), and a
 //    wave multiplies no fragment past K: widening a KiB of bytes takes a SIMD about 100 clocks.
 // For the same reason a weight with few tiles (N = 1536: 96 of 16 rows on 256 CUs) is dealt in halves
-// (wide down 12288 x 1536: 9.6 us in whole tiles, 7.0 in halves): with HALF a unit is 8 weight rows, and a fragment load takes them from two
+// (wide down 12288 x 1536: 9.6 us in whole tiles, 6.8 in halves): with HALF a unit is 8 weight rows, and a fragment load takes them from two
 // k-blocks at once: lane l holds row l % 8 of the unit, of k-block 2 q + (l % 16 >= 8) for pair q,
 // bytes 16 (l / 16).  The MFMA's column 0 gets the activations of the even k-block and column 1
 // those of the odd one, so the sums of rows 0..7 of column 0 and rows 8..15 of column 1 are the
-// unit's two parts, added first when the waves' partials are.  Without HALF, a GELU pair (ACT 1) is
-// 8 gate rows and the same 8 up rows in one tile, from the two fragments that hold them.
-// The order of every sum follows from (N, K) alone, so the plain GEMV, the activations and the
-// prologues agree bit for bit.
-template <int U, bool PACKED, int ACT, int PRO, bool HALF>
+// unit's two partial sums.  Without HALF, a GELU pair (ACT 1) is 8 gate rows and the same 8 up rows in
+// one tile, from the two fragments that hold them.
+// The order of every sum is that of gemv_kernel for the same (N, K), so a row gives the same bits alone
+// and among 2..16, and so do the plain GEMV, the activations and the prologues: few_tile_split partial
+// sums, number v over the k-blocks v, v + parts, .., added in order.  A wave makes the R numbered ks and
+// ks + split in turn (parts = R * split), or with HALF, R = 1, the two numbered 2 ks and 2 ks + 1.
+template <int U, bool PACKED, int ACT, int PRO, bool HALF, int R>
 __global__ __launch_bounds__(PRO == 4 ? 1024 : 768) void gemv1_kernel(GemvParams p) {
   constexpr bool NORM = PRO <= 3;                  // PRO chunks of 512 (K <= 1536)
   constexpr int XS = PRO == 5 ? GEMV_ROW_MAX : PRO == 4 ? 4096 : PRO * 512;
   constexpr int TPW = ACT == 1 && HALF ? 2 : 1;    // HALF pairs: the gate rows' and the up rows' fragments
   constexpr bool SPLIT_ROWS = HALF || ACT == 1;    // a unit is 8 output columns
   constexpr bool PAIR = ACT == 1 && !HALF;         // gate and up rows in one fragment
-  __shared__ v4f red[16][TPW][4];                  // per wave: rows 4j .. 4j+3 of its tile
+  static_assert(!HALF || R == 1, "HALF's two sums are two columns of one accumulator");
+  static_assert(R == 1 || U % 2 == 0 || U <= 3, "a wave's steps alternate; odd U only where one round is all");
+  __shared__ v4f red[32][TPW][4];                  // per partial sum of the workgroup: rows 4j .. 4j+3 of its tile
   __shared__ __attribute__((aligned(16))) uint16_t xs[XS + 16];               // the row, and a piece of zeros
   __shared__ __attribute__((aligned(16))) uint16_t hs[NORM ? PRO * 512 : 8];  // NORM: the first norm's row
   __shared__ float mw[PRO == 4 ? MERGE_HEADS * (DEC_MERGE_IN_GEMV_CHUNKS + 1) : 1];  // PRO 4: chunk weights
@@ -480,6 +484,7 @@ __global__ __launch_bounds__(PRO == 4 ? 1024 : 768) void gemv1_kernel(GemvParams
   const int split = p.split;
   const int gib = wave / split, ks = wave % split;
   const int unit = int(blockIdx.x) * p.gpb + gib;
+  const int parts = (HALF ? 2 : R) * split;  // partial sums of a unit
   const bool active = gib < p.gpb && unit < p.units;
   const int i = lane & 15, j = lane >> 4;  // fragment row and 16-byte chunk
 
@@ -549,9 +554,11 @@ __global__ __launch_bounds__(PRO == 4 ? 1024 : 768) void gemv1_kernel(GemvParams
   const bool column = i < (HALF ? 2 : 1);
   const uint16_t* const xbase = column ? xs + (HALF ? i * 64 : 0) + j * 16 : xs + XS;
   const int xstep = column ? (HALF ? 128 : 64) : 0;
-  v4f acc[TPW];
+  v4f acc[R][TPW];
 #pragma unroll
-  for (int t = 0; t < TPW; ++t) acc[t] = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int r = 0; r < R; ++r)
+#pragma unroll
+    for (int t = 0; t < TPW; ++t) acc[r][t] = v4f{0.f, 0.f, 0.f, 0.f};
   for (int st0 = ks; st0 < nstep; st0 += split * U) {
     if (st0 != ks) {
 #pragma unroll
@@ -564,37 +571,50 @@ __global__ __launch_bounds__(PRO == 4 ? 1024 : 768) void gemv1_kernel(GemvParams
       const uint16_t* xv = xbase + st * xstep;
       const v4i xa = *reinterpret_cast<const v4i*>(xv), xb = *reinterpret_cast<const v4i*>(xv + 8);
 #pragma unroll
-      for (int t = 0; t < TPW; ++t) acc[t] = mma_block(wv[u][t], xa, xb, acc[t]);
+      for (int t = 0; t < TPW; ++t) acc[u % R][t] = mma_block(wv[u][t], xa, xb, acc[u % R][t]);
     }
   }
 
-  // Partials: lane 16 j + c holds rows 4j .. 4j+3 of column c; HALF's rows 8.. belong to column 1.
-  if (i == (HALF && j >= 2 ? 1 : 0)) {
+  // Partials: lane 16 j + c holds rows 4j .. 4j+3 of column c; HALF's rows 8.. of column 1 are rows 0..
+  // of the odd k-blocks.
+  if (active && i == (HALF && j >= 2 ? 1 : 0)) {
 #pragma unroll
-    for (int t = 0; t < TPW; ++t) red[wave][t][j] = acc[t];
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int t = 0; t < TPW; ++t) {
+        if constexpr (HALF) red[2 * wave + (j >> 1)][t][j & 1] = acc[r][t];
+        else red[gib * parts + ks + r * split][t][j] = acc[r][t];
+      }
   }
   __syncthreads();
   if (ks != 0 || !active) return;
-  // Lanes 16 j add the group's partials of rows 4j .. wave by wave; lanes 0 and 16 then take rows 8..
-  // (with HALF the same columns' other part, in a PAIR their up sums) from lanes 32 and 48.
+  // Lanes 16 j add the unit's partials of rows 4j .. in order; in a PAIR lanes 0 and 16 then take their
+  // columns' up sums, rows 8.., from lanes 32 and 48.
   v4f sum[TPW], other[TPW];
 #pragma unroll
   for (int t = 0; t < TPW; ++t) {
-    // sixteen reads without a branch; those past the group are another wave's and left out
-    v4f part[16];
+    // eight at a time, read without a branch; those past the unit are another's and left out
+    v4f part[8], more[8];
 #pragma unroll
-    for (int q = 0; q < 16; ++q) part[q] = red[(wave + q) & 15][t][j];
+    for (int q = 0; q < 8; ++q) part[q] = red[(gib * parts + q) & 31][t][j];
+    if constexpr (HALF || R == 2) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) more[q] = red[(gib * parts + 8 + q) & 31][t][j];
+    }
     sum[t] = part[0];
 #pragma unroll
-    for (int q = 1; q < 16; ++q) {
+    for (int q = 1; q < 8; ++q) {
       const v4f s = sum[t] + part[q];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) sum[t][r] = q < split ? s[r] : sum[t][r];
+      for (int r = 0; r < 4; ++r) sum[t][r] = q < parts ? s[r] : sum[t][r];
     }
-    if constexpr (SPLIT_ROWS) {
+    if ((HALF || R == 2) && parts == 16) {
+#pragma unroll
+      for (int q = 0; q < 8; ++q) sum[t] += more[q];
+    }
+    if constexpr (PAIR) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) other[t][r] = __shfl_xor(sum[t][r], 32, 64);
-      if constexpr (HALF) sum[t] += other[t];
     }
   }
   if (i != 0 || (SPLIT_ROWS && j >= 2)) return;
@@ -660,22 +680,24 @@ static void gemv_launch_few(const GemvParams& p, int64_t groups, hipStream_t str
   }
 }
 
-// One row: HALF where the 16-row tiles would leave half of the CUs without one.  A unit's K range is
-// split over 8 waves while a CU has one unit (HALF, or N <= 4096 on 256 CUs), over 4 from two units
-// per CU on: the waves of a CU then stand evenly on its four SIMDs (3 or 6 waves per unit cost the
-// gate/up GEMV 1-2 us more), and more waves only add partials (down 6144 x 1536 in halves: 16 waves
-// 5.5 us, 8 waves 4.8, 6 waves 5.5).  The split depends on (N, K) alone; the units per
+// One row: HALF where the 16-row tiles would leave half of the CUs without one.  A unit's few_tile_split
+// partial sums are shared by up to 8 waves while a CU has one unit (HALF, or N <= 4096 on 256 CUs), by
+// up to 4 from two units per CU on: the waves of a CU then stand evenly on its four SIMDs (3 or 6 waves per
+// unit cost the gate/up GEMV 1-2 us more), and more waves only cost barriers (down 6144 x 1536 in halves:
+// 16 waves 5.5 us, 8 waves 4.7, 6 waves 5.5).  The partial sums depend on (N, K) alone; the units per
 // workgroup, which change no sum, are one, or with a row to make (the norm, the merge) up to three,
 // so that the row is made less often (gate/up 1536 x 12288: 8.4 us with one, 7.5 with three).
-static bool gemv1_plan(GemvParams& p, bool make_row) {
+// Sets units, split and gpb; the kernel's R, or 0 for HALF.
+static int gemv1_plan(GemvParams& p, bool make_row) {
   const int cus = gemv_cu_count();
   const int ntiles = (p.N + 15) / 16;
   const bool half = 2 * ntiles <= cus;
   const int per_cu = half ? 1 : (ntiles + cus - 1) / cus;
+  const int parts = few_tile_split(ntiles, p.KB);  // a power of two, above 8 only at one unit per CU
   p.units = half ? (p.N + 7) / 8 : ntiles;
-  p.split = min(per_cu == 1 ? 8 : 4, half ? (p.KB + 1) / 2 : p.KB);
+  p.split = half ? max(parts / 2, 1) : min(per_cu == 1 ? 8 : 4, parts);
   p.gpb = make_row ? min(per_cu, 3) : 1;
-  return half;
+  return half ? 0 : parts / p.split;
 }
 
 // Whether a call takes the one-row kernel: its row fits in LDS and its tiles are few.
@@ -686,17 +708,19 @@ static bool gemv1_takes(const GemvParams& p) {
 // U fragments in flight per wave: all of a wave's share in one round where the registers allow it.
 // MI355X, weights cold, a chain of launches replayed from a graph (a chain of empty ones takes 1.9 us
 // each), us per launch, before (one tile per workgroup of 8 or 16 waves, the row made by one wave, the
-// scales fetched after the sums) -> now: o 2048 x 1536 4.5 -> 3.4, 4096 x 1536 5.5 -> 4.2; qkv 1536 x
-// 2560 with its norm 6.3 -> 4.6; gate/up with norm and GELU 1536 x 12288 10.6 -> 7.0, x 24576 13.8 ->
-// 10.9; down 6144 x 1536 7.0 -> 4.9, 12288 x 1536 10.5 -> 7.0; per-layer gate 1536 x 256 with norm
-// 6.3 -> 4.5, projection 256 x 1536 3.3 -> 3.0.  (4.8, 7.7, 12.1 for the qkv and gate/up rows before the
-// packed widening and the branch-free row reads.)
+// scales fetched after the sums) -> now: o 2048 x 1536 4.5 -> 3.3, 4096 x 1536 5.5 -> 4.0; qkv 1536 x
+// 2560 with its norm 6.3 -> 4.4; gate/up with norm and GELU 1536 x 12288 10.5 -> 6.9, x 24576 13.8 ->
+// 10.6; down 6144 x 1536 7.0 -> 4.7, 12288 x 1536 10.5 -> 6.8; per-layer gate 1536 x 256 with norm
+// 6.3 -> 4.4, projection 256 x 1536 3.3 -> 2.8.  (gate/up x 12288 and x 24576: 0.7 and 1.2 more before the
+// packed widening and the branch-free row reads.  x 24576 needs its 80 registers, two workgroups of 12
+// waves per CU: 13.0 at 85.)
 template <bool PACKED, int ACT, int PRO>
 static void gemv1_launch(const GemvParams& p0, hipStream_t stream) {
   GemvParams p = p0;
   // ACT 1 deals the same number of units of 8 gate and 8 up rows as the plain launch of N has
   // tiles, so its sums are made in the same order
-  const bool half = gemv1_plan(p, PRO != 5);
+  const int R = gemv1_plan(p, PRO != 5);
+  const bool half = R == 0;
   // The merge reads every chunk's partials (64 KiB at 8 chunks of 8 heads of 256): both halves of a tile in
   // one workgroup make the row half as often (o projection 2048 x 1536, 8 chunks: 8.1 -> 7.3 us).
   if (PRO == 4 && half) p.gpb = 2;
@@ -705,17 +729,19 @@ static void gemv1_launch(const GemvParams& p0, hipStream_t stream) {
   const dim3 grid(unsigned((p.units + p.gpb - 1) / p.gpb)), block(unsigned(waves * 64));
   const int steps = half ? (p.KB + 1) / 2 : p.KB;
   const int per_wave = (steps + p.split - 1) / p.split;
-#define W8A8_GEMV1(U)                                                                   \
-  do {                                                                                  \
-    if (half) gemv1_kernel<U, PACKED, ACT, PRO, true><<<grid, block, 0, stream>>>(p);   \
-    else gemv1_kernel<U, PACKED, ACT, PRO, false><<<grid, block, 0, stream>>>(p);       \
+#define W8A8_GEMV1(U)                                                                                      \
+  do {                                                                                                     \
+    if (half) gemv1_kernel<U, PACKED, ACT, PRO, true, 1><<<grid, block, 0, stream>>>(p);                   \
+    else if (R == 2) gemv1_kernel<U, PACKED, ACT, PRO, false, 2><<<grid, block, 0, stream>>>(p);           \
+    else gemv1_kernel<U, PACKED, ACT, PRO, false, 1><<<grid, block, 0, stream>>>(p);                       \
   } while (0)
   if (per_wave <= 1) W8A8_GEMV1(1);
   else if (per_wave <= 2) W8A8_GEMV1(2);
   else if (per_wave <= 3) W8A8_GEMV1(3);
   else if (per_wave <= 4 || (ACT == 1 && half)) W8A8_GEMV1(4);
   else if (per_wave <= 6 || half || PRO == 4) W8A8_GEMV1(6);
-  else gemv1_kernel<PRO == 4 ? 6 : 12, PACKED, ACT, PRO, false><<<grid, block, 0, stream>>>(p);
+  else if (R == 2) gemv1_kernel<PRO == 4 ? 6 : 12, PACKED, ACT, PRO, false, 2><<<grid, block, 0, stream>>>(p);
+  else gemv1_kernel<PRO == 4 ? 6 : 12, PACKED, ACT, PRO, false, 1><<<grid, block, 0, stream>>>(p);
 #undef W8A8_GEMV1
 }
 

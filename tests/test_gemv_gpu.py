@@ -355,3 +355,26 @@ def test_gemv_one_row_gelu_pair_and_norm_agree(I, K):
     assert torch.equal(gh, h) and torch.equal(got, ops.gelu_mul_bf16(ops.gemv_bf16(x, pw, s)))
     got, _ = ops.gemv_norm_bf16(y, r, w1, 1e-6, pw, s, w2=w2)
     assert torch.equal(got, ops.gemv_bf16(x, pw, s))
+
+
+@pytest.mark.parametrize("N, K", ONE_ROW + [(1, 16), (256, 1536), (1536, 256), (2560, 1536), (5120, 1536), (1536, 6144),
+                                            (12288, 1536), (24576, 1536), (33000, 320), (4096, 12288)])
+def test_gemv_a_row_has_the_same_bits_alone_and_among_others(N, K):
+    """One row takes a kernel of its own, with the sums of the kernel of 2..16 rows in the same order: row 0 of
+    a call of five rows equals a call of row 0, bit for bit, packed and row-major, plain, GELU pair and GELU
+    times a multiplier.  The second half of K repeats the first with nearly the opposite activations, so that
+    the sums cancel and another order of the same fp32 terms shows in bf16."""
+    g = torch.Generator(device=DEV).manual_seed(N * 5 + K)
+    x = torch.randn(5, K, generator=g, device=DEV).to(torch.bfloat16)
+    w = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8, device=DEV)
+    h = K // 32 * 16
+    x[:, h:2 * h] = -x[:, :h] * (1 + torch.randn(5, h, generator=g, device=DEV) / 256).to(torch.bfloat16)
+    w[:, h:2 * h] = w[:, :h]
+    s = torch.rand(N, generator=g, device=DEV) * 0.01
+    mul = torch.randn(5, N, generator=g, device=DEV).to(torch.bfloat16)
+    pw = ops.pack_gemv_weight(w)
+    print(f"a row alone and among five: N={N} K={K}", flush=True)
+    for call in (lambda r: ops.gemv_bf16(x[:r], pw, s), lambda r: ops.gemv_bf16(x[:r], w, s),
+                 lambda r: ops.gemv_act_bf16(x[:r], pw, s, "gelu_mul", mul=mul[:r]),
+                 *([lambda r: ops.gemv_act_bf16(x[:r], pw, s, "gelu_pair")] if N % 32 == 0 else [])):
+        assert torch.equal(call(1), call(5)[:1])
