@@ -10,7 +10,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import assert_bf16_close, f32, to_bits
+from helpers import assert_bf16_close, f32, from_bits, to_bits
 
 import oracle.oracle as orc
 from w8a8 import fused, ops, workloads
@@ -256,6 +256,15 @@ def test_row_kernels_at_other_hidden_sizes(N):
 
 
 # ---- k_gelu / k_ple_gate ------------------------------------------------------------------
+
+def test_gelu_of_every_bf16_value():
+    """GELU alone (times 1) of all 65280 finite bf16 values, as 255 rows, against the oracle's: the same bits."""
+    b = np.arange(65536, dtype=np.uint16)
+    b = b[(b & 0x7f80) != 0x7f80].reshape(255, 256)
+    one = np.full_like(b, 0x3f80)
+    got = ops.gelu_mul_bf16(from_bits(b).to(DEV), from_bits(one).to(DEV))
+    assert np.array_equal(to_bits(got), orc.gelu_mul(np.concatenate([b, one], 1)))
+
 
 @pytest.mark.parametrize("T,I", [(33, 6144), (5, 256)])
 def test_k_gelu(T, I):
