@@ -261,10 +261,9 @@ __device__ __forceinline__ v4i load_weight(__amdgpu_buffer_rsrc_t r, uint32_t of
 }
 
 // The epilogue's operands of one lane: for T tiles `tstep` columns apart, the scales of columns n0 ..
-// n0+3, and for ACT 2 row m's multipliers.  load() only asks for them, bounds-checked and without a
+// n0+3, and for ACT 2 row m's multipliers.  load() only asks for them, kept in bounds without a
 // branch or a conversion per element (either would wait for the element before the next is asked
-// for: 3 us of the gate/up GEMV); scale() and mul() convert.  Columns past N read zero and are not
-// stored.
+// for: 3 us of the gate/up GEMV); scale() and mul() convert.  Columns past N are not stored.
 template <int T, int ACT>
 struct GemvScales {
   uint32_t s[T][4], m[4];
@@ -285,10 +284,11 @@ struct GemvScales {
           s[t][r] = __builtin_amdgcn_raw_buffer_load_b16(rs, uint32_t(n0 + t * tstep + r) * 2u, 0, 0);
     }
     if constexpr (ACT == 2) {
-      const __amdgpu_buffer_rsrc_t rm = make_rsrc(p.mul, uint32_t(((p.M - 1) * p.ldm + p.N) * 2));
+      // rows have a 64-bit base each (ldm may be any stride); the last row and column stand for those past
+      // them, whose results are not stored
+      const uint16_t* const mr = p.mul + int64_t(min(row, p.M - 1)) * p.ldm;
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        m[r] = __builtin_amdgcn_raw_buffer_load_b16(rm, row < p.M ? uint32_t(row * p.ldm + n0 + r) * 2u : 0x80000000u, 0, 0);
+      for (int r = 0; r < 4; ++r) m[r] = mr[min(n0 + r, p.N - 1)];
     }
   }
   __device__ __forceinline__ float scale(const GemvParams& p, int t, int r) const {

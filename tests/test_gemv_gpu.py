@@ -241,6 +241,21 @@ def test_gemv_gelu_mul_equals_gemv_then_gelu_mul(M, K, N):
         ops.gemv_act_bf16(x, pw, s, "gelu_mul")
 
 
+@pytest.mark.parametrize("M, ldm", [(2, 2 ** 31), (5, 2 ** 29 + 8), (16, 2 ** 31 // 15 + 1)])
+def test_gemv_gelu_mul_rows_beyond_32_bits(M, ldm):
+    """Multiplier rows whose last one lies 2^31 elements (4 GiB) or more after the first."""
+    K, N = 64, 48
+    g = torch.Generator(device=DEV).manual_seed(M)
+    x = torch.randn(M, K, generator=g, device=DEV).to(torch.bfloat16)
+    pw = ops.pack_gemv_weight(torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8, device=DEV))
+    s = torch.rand(N, generator=g, device=DEV) * 0.01
+    rows = torch.randn(M, N, generator=g, device=DEV).to(torch.bfloat16)
+    mul = torch.empty((M - 1) * ldm + N, dtype=torch.bfloat16, device=DEV).as_strided((M, N), (ldm, 1))
+    mul.copy_(rows)
+    want = ops.gelu_mul_bf16(ops.gemv_bf16(x, pw, s), rows)
+    assert torch.equal(ops.gemv_act_bf16(x, pw, s, "gelu_mul", mul=mul), want)
+
+
 @pytest.mark.parametrize("K, N, act", [(1536, 2560, None), (1536, 2 * 6144, "gelu_pair"), (1536, 256, "gelu_mul"),
                                        (256, 640, None), (1024, 96, "gelu_pair"), (1296, 200, None)])
 def test_gemv_norm_equals_row_kernel_then_gemv(K, N, act):
