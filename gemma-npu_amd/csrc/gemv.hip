@@ -662,7 +662,7 @@ static int few_tile_split(int64_t ntiles, int KB) {
   return split;
 }
 
-// The few-tile launch of 2..16 rows: per tile group `split` waves, NWB = split for 8 and 16.
+// The few-tile launch of what gemv1_takes leaves: per tile group `split` waves, NWB = split for 8 and 16.
 template <bool PACKED, int TPW, int ACT>
 static void gemv_launch_few(const GemvParams& p, int64_t groups, hipStream_t stream) {
   const int per_wave = (p.KB + p.split - 1) / p.split;
@@ -685,8 +685,8 @@ static void gemv_launch_few(const GemvParams& p, int64_t groups, hipStream_t str
 // up to 4 from two units per CU on: the waves of a CU then stand evenly on its four SIMDs (3 or 6 waves per
 // unit cost the gate/up GEMV 1-2 us more), and more waves only cost barriers (down 6144 x 1536 in halves:
 // 16 waves 5.5 us, 8 waves 4.7, 6 waves 5.5).  The partial sums depend on (N, K) alone; the units per
-// workgroup, which change no sum, are one, or with a row to make (the norm, the merge) up to three,
-// so that the row is made less often (gate/up 1536 x 12288: 8.4 us with one, 7.5 with three).
+// workgroup, which change no sum, are one, or with a row to make (the norm, the merge) up to twelve waves'
+// worth, so that the row is made less often (gate/up 1536 x 12288: 8.4 us with one, 7.5 with three).
 // Sets units, split and gpb; the kernel's R, or 0 for HALF.
 static int gemv1_plan(GemvParams& p, bool make_row) {
   const int cus = gemv_cu_count();
@@ -696,16 +696,22 @@ static int gemv1_plan(GemvParams& p, bool make_row) {
   const int parts = few_tile_split(ntiles, p.KB);  // a power of two, above 8 only at one unit per CU
   p.units = half ? (p.N + 7) / 8 : ntiles;
   p.split = half ? max(parts / 2, 1) : min(per_cu == 1 ? 8 : 4, parts);
-  p.gpb = make_row ? min(per_cu, 3) : 1;
+  p.gpb = make_row ? min(per_cu, 12 / p.split) : 1;
   return half ? 0 : parts / p.split;
 }
 
-// Whether a call takes the one-row kernel: its row fits in LDS and its tiles are few.
+// Whether a call takes the one-row kernel: its row fits in LDS, and its tiles are few.  From 2048 tiles
+// on a tile has one or two partial sums, and a workgroup of as many waves copying the row into LDS again
+// costs more than it saves: N x K 50000 x 64 6.0 us here, 3.8 in gemv_kernel; 33000 x 256 5.1 and 4.4;
+// 32768 x 1536 12.5 and 12.0; 65000 x 1536 the same.  Below, 20000 x 64 3.1 us here, 3.5 there before.
 static bool gemv1_takes(const GemvParams& p) {
-  return p.M == 1 && p.KB * 64 <= GEMV_ROW_MAX && (int64_t(p.N) + 15) / 16 < 4096;
+  return p.M == 1 && p.KB * 64 <= GEMV_ROW_MAX && (int64_t(p.N) + 15) / 16 < 2048;
 }
 
-// U fragments in flight per wave: all of a wave's share in one round where the registers allow it.
+// U fragments in flight per wave: all of a wave's share in one round where the registers allow it (seven or
+// eight steps in one round of 8 rather than 12: 4096 x 4096 6.4 -> 6.1 us, row-major 7.4 -> 7.0, N = 16384,
+// K = 2048 9.6 -> 8.5).  With the norm six at most, whose 80 registers let two workgroups of twelve waves
+// stand on a CU (N = 32768, K = 1536, two waves per unit: 18.2 us in rounds of 12, 14.2 in rounds of 6).
 // MI355X, weights cold, a chain of launches replayed from a graph (a chain of empty ones takes 1.9 us
 // each), us per launch, before (one tile per workgroup of 8 or 16 waves, the row made by one wave, the
 // scales fetched after the sums) -> now: o 2048 x 1536 4.5 -> 3.3, 4096 x 1536 5.5 -> 4.0; qkv 1536 x
@@ -729,20 +735,25 @@ static void gemv1_launch(const GemvParams& p0, hipStream_t stream) {
   const dim3 grid(unsigned((p.units + p.gpb - 1) / p.gpb)), block(unsigned(waves * 64));
   const int steps = half ? (p.KB + 1) / 2 : p.KB;
   const int per_wave = (steps + p.split - 1) / p.split;
-#define W8A8_GEMV1(U)                                                                                      \
-  do {                                                                                                     \
-    if (half) gemv1_kernel<U, PACKED, ACT, PRO, true, 1><<<grid, block, 0, stream>>>(p);                   \
-    else if (R == 2) gemv1_kernel<U, PACKED, ACT, PRO, false, 2><<<grid, block, 0, stream>>>(p);           \
-    else gemv1_kernel<U, PACKED, ACT, PRO, false, 1><<<grid, block, 0, stream>>>(p);                       \
+#define W8A8_GEMV1_WHOLE(U)                                                                      \
+  do {                                                                                           \
+    if (R == 2) gemv1_kernel<U, PACKED, ACT, PRO, false, 2><<<grid, block, 0, stream>>>(p);      \
+    else gemv1_kernel<U, PACKED, ACT, PRO, false, 1><<<grid, block, 0, stream>>>(p);             \
+  } while (0)
+#define W8A8_GEMV1(U)                                                                            \
+  do {                                                                                           \
+    if (half) gemv1_kernel<U, PACKED, ACT, PRO, true, 1><<<grid, block, 0, stream>>>(p);         \
+    else W8A8_GEMV1_WHOLE(U);                                                                    \
   } while (0)
   if (per_wave <= 1) W8A8_GEMV1(1);
   else if (per_wave <= 2) W8A8_GEMV1(2);
   else if (per_wave <= 3) W8A8_GEMV1(3);
   else if (per_wave <= 4 || (ACT == 1 && half)) W8A8_GEMV1(4);
-  else if (per_wave <= 6 || half || PRO == 4) W8A8_GEMV1(6);
-  else if (R == 2) gemv1_kernel<PRO == 4 ? 6 : 12, PACKED, ACT, PRO, false, 2><<<grid, block, 0, stream>>>(p);
-  else gemv1_kernel<PRO == 4 ? 6 : 12, PACKED, ACT, PRO, false, 1><<<grid, block, 0, stream>>>(p);
+  else if (per_wave <= 6 || half || PRO != 5) W8A8_GEMV1(6);
+  else if (per_wave <= 8) W8A8_GEMV1_WHOLE(8);
+  else W8A8_GEMV1_WHOLE(PRO != 5 ? 8 : 12);
 #undef W8A8_GEMV1
+#undef W8A8_GEMV1_WHOLE
 }
 
 template <bool PACKED>

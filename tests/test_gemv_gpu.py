@@ -373,7 +373,8 @@ def test_gemv_one_row_gelu_pair_and_norm_agree(I, K):
 
 
 @pytest.mark.parametrize("N, K", ONE_ROW + [(1, 16), (256, 1536), (1536, 256), (2560, 1536), (5120, 1536), (1536, 6144),
-                                            (12288, 1536), (24576, 1536), (33000, 320), (4096, 12288)])
+                                            (12288, 1536), (24576, 1536), (33000, 320), (4096, 12288),
+                                            (32752, 48), (32768, 48), (4096, 4096), (4096, 3136), (16384, 2048), (30000, 1600)])
 def test_gemv_a_row_has_the_same_bits_alone_and_among_others(N, K):
     """One row takes a kernel of its own, with the sums of the kernel of 2..16 rows in the same order: row 0 of
     a call of five rows equals a call of row 0, bit for bit, packed and row-major, plain, GELU pair and GELU
