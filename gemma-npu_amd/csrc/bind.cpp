@@ -5,9 +5,10 @@
 // Every function takes the wrapper's tensors, checks the plain case (exact torch.Tensor, GPU, dtype,
 // rank, contiguous rows, one device, matching shapes), allocates the outputs, calls the C ABI on
 // torch's current stream of that device with the GIL released, and returns the outputs.  Anything else
-// -- another type, a mismatch, an allocation or a launch that fails -- returns None without having
-// launched anything, and the wrapper's own code then runs the call or raises its error: this path
-// accepts nothing that the wrapper refuses and words no error itself.
+// -- another type, a mismatch, an allocation that fails, a status that the C entry decides before its
+// outputs are touched -- returns None, and the wrapper's own code then runs the call or raises its error:
+// this path accepts nothing that the wrapper refuses.  W8A8_EHIP comes from after a launch, or clears an
+// earlier call's error, so it is raised here as the wrappers raise it, and nothing is run again.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -16,7 +17,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <algorithm>
-#include <exception>
+#include <string>
 
 #include "w8a8.h"
 
@@ -31,6 +32,13 @@ struct Decline {};
 void need(bool ok) {
   if (!ok) throw Decline{};
 }
+
+// A C entry that failed with its work possibly queued.
+struct Failed {
+  std::string fn;
+  int rc;
+  std::string msg;
+};
 
 // The device of a call, fixed by its first tensor; every other one must be on it.
 struct Call {
@@ -96,14 +104,27 @@ float real(PyObject* o) {
   return static_cast<float>(v);
 }
 
-// Runs a C entry with the GIL released; a status other than W8A8_OK declines (nothing was launched).
+// Runs the C entry `fn` with the GIL released.
 template <class F>
-void launch(F&& f) {
+void launch(const char* fn, F&& f) {
   int rc;
   Py_BEGIN_ALLOW_THREADS
   rc = f();
   Py_END_ALLOW_THREADS
-  need(rc == W8A8_OK);
+  if (rc == W8A8_EINVAL || rc == W8A8_EALIGN || rc == W8A8_ENOTSUP) throw Decline{};
+  if (rc != W8A8_OK) throw Failed{fn, rc, w8a8_last_error()};
+}
+
+// Raises w8a8._lib.W8A8Error, as _lib.call does.
+PyObject* raise_failed(const Failed& e) {
+  PyObject* m = PyImport_ImportModule("w8a8._lib");
+  PyObject* cls = m ? PyObject_GetAttrString(m, "W8A8Error") : nullptr;
+  PyObject* err = cls ? PyObject_CallFunction(cls, "sis", e.fn.c_str(), e.rc, e.msg.c_str()) : nullptr;
+  if (err) PyErr_SetObject(cls, err);
+  Py_XDECREF(err);
+  Py_XDECREF(cls);
+  Py_XDECREF(m);
+  return nullptr;
 }
 
 PyObject* none() { Py_RETURN_NONE; }
@@ -138,7 +159,7 @@ PyObject* gemv(PyObject* const* a) {
   need(s.size(0) == N);
   const Tensor y = output(c, a[5], M, N, at::kBFloat16);
   const hipStream_t st = c.stream();
-  launch([&] {
+  launch("w8a8_gemv_packed_bf16", [&] {
     return w8a8_gemv_packed_bf16(bf(x), ld(x), M, i8(w), N, K, s.data_ptr(), sd == at::kFloat ? 1 : 0, bfo(y), ld(y), st);
   });
   return wrap(y);
@@ -170,7 +191,7 @@ PyObject* linear(PyObject* const* a) {
   const Tensor ws = a[11] != Py_None ? c.vec(a[11], at::kByte)
                                      : c.make({std::max<int64_t>(w8a8_linear_workspace_bytes(M, N, K), 256)}, at::kByte);
   const hipStream_t st = c.stream();
-  launch([&] {
+  launch("w8a8_linear_bf16", [&] {
     return w8a8_linear_bf16(bf(x), ld(x), i8(w), f32(sw), M, N, K, int(epi), I, res, ldr, rw, eps, bfo(y), ld(y),
                             ws.data_ptr(), ws.numel(), st);
   });
@@ -201,7 +222,7 @@ PyObject* gemm_i32(PyObject* const* a) {
   need(A.K == integer(a[5]));
   const Tensor y = output(c, a[6], A.M, N, at::kInt);
   const hipStream_t st = c.stream();
-  launch([&] {
+  launch("w8a8_gemm_i32_ex", [&] {
     return w8a8_gemm_i32_ex(A.p, A.lda, A.packed, i8(w), A.M, N, A.K, static_cast<int32_t*>(y.data_ptr()), ld(y), -1, 0,
                             nullptr, 0, st);
   });
@@ -229,7 +250,7 @@ PyObject* gemm_bf16(PyObject* const* a) {
   }
   const Tensor y = output(c, a[11], A.M, epi == 1 ? I : N, at::kBFloat16);
   const hipStream_t st = c.stream();
-  launch([&] {
+  launch("w8a8_gemm_bf16_ex", [&] {
     return w8a8_gemm_bf16_ex(A.p, A.lda, A.packed, f32(sx), i8(w), f32(sw), A.M, N, A.K, int(epi), I, res, ldr, bfo(y),
                              ld(y), -1, 0, nullptr, 0, st);
   });
@@ -249,7 +270,7 @@ PyObject* quant_packed(PyObject* const* a) {
   const int64_t M = x.size(0), K = x.size(1);
   const Tensor q = packed_rows(c, M, K), s = c.make({M}, at::kFloat);
   const hipStream_t st = c.stream();
-  launch([&] { return w8a8_quant_rows_packed_bf16(bf(x), ld(x), M, K, i8(q), f32(s), st); });
+  launch("w8a8_quant_rows_packed_bf16", [&] { return w8a8_quant_rows_packed_bf16(bf(x), ld(x), M, K, i8(q), f32(s), st); });
   return tuple(q, s);
 }
 
@@ -262,7 +283,7 @@ PyObject* k_in(PyObject* const* a) {
   const float eps = real(a[2]);
   const Tensor q = packed_rows(c, M, N), s = c.make({M}, at::kFloat);
   const hipStream_t st = c.stream();
-  launch([&] { return w8a8_k_in(bf(h), ld(h), w, eps, M, N, i8(q), 0, 1, f32(s), st); });
+  launch("w8a8_k_in", [&] { return w8a8_k_in(bf(h), ld(h), w, eps, M, N, i8(q), 0, 1, f32(s), st); });
   return tuple(q, s);
 }
 
@@ -301,7 +322,7 @@ PyObject* k_post_attn(PyObject* const* a) {
   const float eps = real(a[6]);
   const Tensor h = c.make({M, N}, at::kBFloat16), q = packed_rows(c, M, N), s = c.make({M}, at::kFloat);
   const hipStream_t st = c.stream();
-  launch([&] {
+  launch(acc.y ? "w8a8_k_post_attn_y" : "w8a8_k_post_attn", [&] {
     return acc.y ? w8a8_k_post_attn_y(acc.rows(), acc.stride(), bf(res), ld(res), w1, w2, eps, M, N, bfo(h), N, i8(q), 0, 1,
                                       f32(s), st)
                  : w8a8_k_post_attn(acc.i32(), acc.stride(), acc.sx, acc.sw, bf(res), ld(res), w1, w2, eps, M, N, bfo(h), N,
@@ -321,7 +342,7 @@ PyObject* k_post_ff(PyObject* const* a) {
   const float eps = real(a[5]);
   const Tensor h = c.make({M, N}, at::kBFloat16), q = packed_rows(c, M, N), s = c.make({M}, at::kFloat);
   const hipStream_t st = c.stream();
-  launch([&] {
+  launch(acc.y ? "w8a8_k_post_ff_y" : "w8a8_k_post_ff", [&] {
     return acc.y ? w8a8_k_post_ff_y(acc.rows(), acc.stride(), bf(res), ld(res), w, eps, M, N, bfo(h), N, i8(q), 0, 1, f32(s),
                                     st)
                  : w8a8_k_post_ff(acc.i32(), acc.stride(), acc.sx, acc.sw, bf(res), ld(res), w, eps, M, N, bfo(h), N, i8(q),
@@ -339,7 +360,7 @@ PyObject* k_ple_gate(PyObject* const* a) {
   need(acc.t->size(0) == M);
   const Tensor q = packed_rows(c, M, N), s = c.make({M}, at::kFloat);
   const hipStream_t st = c.stream();
-  launch([&] {
+  launch(acc.y ? "w8a8_k_ple_gate_y" : "w8a8_k_ple_gate", [&] {
     return acc.y ? w8a8_k_ple_gate_y(acc.rows(), acc.stride(), bf(ple), ld(ple), M, N, i8(q), 0, 1, f32(s), st)
                  : w8a8_k_ple_gate(acc.i32(), acc.stride(), acc.sx, acc.sw, bf(ple), ld(ple), M, N, i8(q), 0, 1, f32(s), st);
   });
@@ -359,7 +380,7 @@ PyObject* k_ple_out_k_in(PyObject* const* a) {
   const float eps = real(a[6]);
   const Tensor o = c.make({M, N}, at::kBFloat16), q = packed_rows(c, M, N), s = c.make({M}, at::kFloat);
   const hipStream_t st = c.stream();
-  launch([&] {
+  launch(acc.y ? "w8a8_k_ple_out_k_in_y" : "w8a8_k_ple_out_k_in", [&] {
     return acc.y ? w8a8_k_ple_out_k_in_y(acc.rows(), acc.stride(), bf(h), ld(h), w, bf(sc), wn, eps, M, N, bfo(o), N, i8(q), 0,
                                          1, f32(s), st)
                  : w8a8_k_ple_out_k_in(acc.i32(), acc.stride(), acc.sx, acc.sw, bf(h), ld(h), w, bf(sc), wn, eps, M, N,
@@ -387,7 +408,7 @@ PyObject* k_qkv(PyObject* const* a) {
   }
   uint16_t *kp = shared ? nullptr : bfo(k), *vp = shared ? nullptr : bfo(v);
   const hipStream_t st = c.stream();
-  launch([&] {
+  launch(acc.y ? "w8a8_k_qkv_y" : "w8a8_k_qkv", [&] {
     return acc.y ? w8a8_k_qkv_y(acc.rows(), acc.stride(), bf(cs), bf(sn), ld(cs), qw, kw, eps, T, H, KV, D, shared ? 1 : 0,
                                 bfo(q), kp, vp, st)
                  : w8a8_k_qkv(acc.i32(), acc.stride(), acc.sx, acc.sw, bf(cs), bf(sn), ld(cs), qw, kw, eps, T, H, KV, D,
@@ -436,7 +457,7 @@ PyObject* attention(PyObject* const* a) {
   const hipStream_t st = c.stream();
   const Tensor* w = cached(c, a[6], st, w8a8_attention_workspace_bytes(H, KV, Tq, Tk, D, start, window));
   const Tensor ws = w ? *w : Tensor();  // held while the GIL is released
-  launch([&] {
+  launch("w8a8_attention_ws_bf16", [&] {
     return w8a8_attention_ws_bf16(bf(*q.t), q.hs, q.rs, bf(*k.t), k.hs, k.rs, bf(*v.t), v.hs, v.rs, H, KV, Tq, Tk, D, start,
                                   window, scale, bfo(o), std::max<int64_t>(Tq, 1) * D, D, nullptr,
                                   w ? ws.data_ptr() : nullptr, w ? ws.numel() : 0, st);
@@ -457,7 +478,7 @@ PyObject* attention_quant(PyObject* const* a) {
   const hipStream_t st = c.stream();
   const Tensor* w = cached(c, a[6], st, w8a8_attention_workspace_bytes(H, KV, Tq, Tk, D, start, window));
   const Tensor ws = w ? *w : Tensor();
-  launch([&] {
+  launch("w8a8_attention_quant_bf16", [&] {
     return w8a8_attention_quant_bf16(bf(*q.t), q.hs, q.rs, bf(*k.t), k.hs, k.rs, bf(*v.t), v.hs, v.rs, H, KV, Tq, Tk, D,
                                      start, window, scale, i8(x), f32(s), w ? ws.data_ptr() : nullptr, w ? ws.numel() : 0,
                                      st);
@@ -479,14 +500,15 @@ PyObject* decode(PyObject* const* a) {
   const int64_t bytes = w8a8_attention_decode_workspace_bytes(H, KV, Tk, D, pos, window);
   need(bytes > 0);
   const Tensor ws = *cached(c, a[6], st, bytes);
-  launch([&] {
+  launch("w8a8_attention_decode_bf16", [&] {
     return w8a8_attention_decode_bf16(bf(q), H > 1 ? q.stride(0) : D, bf(*k.t), k.hs, k.rs, bf(*v.t), v.hs, v.rs, H, KV, Tk,
                                       D, pos, window, scale, bfo(o), D, nullptr, ws.data_ptr(), ws.numel(), st);
   });
   return wrap(o);
 }
 
-// Waits for torch's current stream of tensor t's device; True when it is done.
+// Waits for torch's current stream of tensor t's device; True when it is done, None without waiting if t is
+// no GPU tensor.
 PyObject* wait_stream(PyObject* const* a) {
   need(THPVariable_CheckExact(a[0]));
   const Tensor& t = THPVariable_Unpack(a[0]);
@@ -498,19 +520,30 @@ PyObject* wait_stream(PyObject* const* a) {
   Py_BEGIN_ALLOW_THREADS
   e = hipStreamSynchronize(st);
   Py_END_ALLOW_THREADS
-  need(e == hipSuccess);
+  if (e != hipSuccess) throw Failed{"hipStreamSynchronize", W8A8_EHIP, hipGetErrorString(e)};
   Py_RETURN_TRUE;
 }
 
-// A METH_FASTCALL entry of `n` arguments around `f`: every refusal and every C++ exception is None.
+// (C entry's name, status) -> what a call whose entry returned it comes to: True, None (declined) or the
+// error raised.
+PyObject* settle(PyObject* const* a) {
+  const char* fn = PyUnicode_AsUTF8(a[0]);
+  need(fn);
+  const int rc = static_cast<int>(integer(a[1]));
+  launch(fn, [&] { return rc; });
+  Py_RETURN_TRUE;
+}
+
+// A METH_FASTCALL entry of `n` arguments around `f`: every refusal and every C++ exception is None, a
+// failed launch is raised.
 template <PyObject* (*f)(PyObject* const*), int n>
 PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
   if (nargs != n) return none();
   try {
     return f(args);
-  } catch (const Decline&) {
-    return none();
-  } catch (const std::exception&) {  // torch's: no storage, out of memory, ...
+  } catch (const Failed& e) {
+    return raise_failed(e);
+  } catch (...) {  // Decline, or torch's: no storage, out of memory, ...
     return none();
   }
 }
@@ -522,6 +555,7 @@ PyMethodDef methods[] = {
     W8A8_ENTRY(quant_packed, 1), W8A8_ENTRY(k_in, 3),           W8A8_ENTRY(k_post_attn, 7), W8A8_ENTRY(k_post_ff, 6),
     W8A8_ENTRY(k_ple_gate, 4),  W8A8_ENTRY(k_ple_out_k_in, 8),  W8A8_ENTRY(k_qkv, 12),    W8A8_ENTRY(attention, 7),
     W8A8_ENTRY(attention_quant, 7), W8A8_ENTRY(decode, 7),      W8A8_ENTRY(wait_stream, 1),
+    W8A8_ENTRY(settle, 2),
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_launch", "The wrappers' launch path in native code.", -1, methods,
                       nullptr, nullptr, nullptr, nullptr};

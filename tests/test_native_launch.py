@@ -5,6 +5,7 @@ gives, and that what the wrapper refuses stays refused with the same error."""
 import pytest
 import torch
 
+import npu_kernels
 from w8a8 import _lib, attention, fused, ops
 
 DEV = "cuda"
@@ -21,6 +22,37 @@ def test_declines_what_it_does_not_take():
     assert n.quant_packed(torch.nn.Parameter(x)) is None
     assert n.attention(x, x, x, 0, 0, 1.0, {}) is None
     assert n.wait_stream(x) is None
+
+
+def test_a_launch_that_fails_is_raised_and_not_run_again(monkeypatch):
+    """Statuses decided before a launch decline; W8A8_EHIP, after which work may be queued, is raised as the
+    wrappers raise it, and the wrapper does not make the call a second time."""
+    n = _lib.launch_module()
+    assert n.settle("w8a8_k_in", _lib.W8A8_OK) is True
+    for status in (_lib.W8A8_EINVAL, _lib.W8A8_EALIGN, _lib.W8A8_ENOTSUP):
+        assert n.settle("w8a8_k_in", status) is None
+    with pytest.raises(_lib.W8A8Error, match="w8a8_k_in: EHIP") as e:
+        n.settle("w8a8_k_in", _lib.W8A8_EHIP)
+    assert e.value.status == _lib.W8A8_EHIP
+
+    class Native:
+        def __getattr__(self, name):
+            return lambda *a: n.settle(f"w8a8_{name}", _lib.W8A8_EHIP)
+
+    def call(*a):
+        raise AssertionError("run again")
+    for m in (ops, fused, attention):
+        monkeypatch.setattr(m, "_native", Native())
+        monkeypatch.setattr(m, "call", call)
+    t, w = torch.zeros(2, 64), ops.PackedWeight(torch.zeros(1), 64, 64, sw=torch.zeros(64))
+    for run in (lambda: ops.gemv_bf16(t, ops.GemvWeight(t, 64, 64), t), lambda: ops.linear_bf16(t, w),
+                lambda: ops.gemm_bf16(t, t, w, epilogue="residual", residual=t, out=t), lambda: ops.gemm_i32(t, w),
+                lambda: ops.quant_rows_packed(t), lambda: fused.k_in(t, t, 1e-6, packed=True),
+                lambda: fused.k_qkv(t, t, t, t, t, t, t, 1e-6, 2, 1, 64, False), lambda: attention.attention(t, t, t),
+                lambda: attention.attention_quant(t, t, t), lambda: attention.decode(t, t, t),
+                lambda: npu_kernels.mm_i8(t, w, t)):
+        with pytest.raises(_lib.W8A8Error, match="EHIP"):
+            run()
 
 
 def both(monkeypatch, call):
