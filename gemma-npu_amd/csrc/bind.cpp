@@ -48,6 +48,7 @@ struct Call {
     need(THPVariable_CheckExact(o));
     const Tensor& t = THPVariable_Unpack(o);
     need(t.is_cuda() && t.layout() == at::kStrided && t.scalar_type() == dt && t.dim() == dim);
+    need(t.has_storage());  // not so inside torch.func's transforms
     if (device < 0) device = t.get_device();
     need(t.get_device() == device);
     return t;
@@ -104,13 +105,20 @@ float real(PyObject* o) {
   return static_cast<float>(v);
 }
 
+// Without the GIL for its lifetime, whichever way its block is left.
+struct Released {
+  PyThreadState* state = PyEval_SaveThread();
+  ~Released() { PyEval_RestoreThread(state); }
+};
+
 // Runs the C entry `fn` with the GIL released.
 template <class F>
 void launch(const char* fn, F&& f) {
   int rc;
-  Py_BEGIN_ALLOW_THREADS
-  rc = f();
-  Py_END_ALLOW_THREADS
+  {
+    Released gil;
+    rc = f();
+  }
   if (rc == W8A8_EINVAL || rc == W8A8_EALIGN || rc == W8A8_ENOTSUP) throw Decline{};
   if (rc != W8A8_OK) throw Failed{fn, rc, w8a8_last_error()};
 }
@@ -517,20 +525,24 @@ PyObject* wait_stream(PyObject* const* a) {
   c.device = t.get_device();
   const hipStream_t st = c.stream();
   hipError_t e;
-  Py_BEGIN_ALLOW_THREADS
-  e = hipStreamSynchronize(st);
-  Py_END_ALLOW_THREADS
+  {
+    Released gil;
+    e = hipStreamSynchronize(st);
+  }
   if (e != hipSuccess) throw Failed{"hipStreamSynchronize", W8A8_EHIP, hipGetErrorString(e)};
   Py_RETURN_TRUE;
 }
 
 // (C entry's name, status) -> what a call whose entry returned it comes to: True, None (declined) or the
-// error raised.
+// error raised.  A negative status throws in the entry's place.
 PyObject* settle(PyObject* const* a) {
   const char* fn = PyUnicode_AsUTF8(a[0]);
   need(fn);
   const int rc = static_cast<int>(integer(a[1]));
-  launch(fn, [&] { return rc; });
+  launch(fn, [&] {
+    if (rc < 0) throw std::string("thrown");
+    return rc;
+  });
   Py_RETURN_TRUE;
 }
 
@@ -543,7 +555,8 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     return f(args);
   } catch (const Failed& e) {
     return raise_failed(e);
-  } catch (...) {  // Decline, or torch's: no storage, out of memory, ...
+  } catch (...) {  // Decline, or torch's: no storage, out of memory, a Python mode's error, ...
+    PyErr_Clear();
     return none();
   }
 }

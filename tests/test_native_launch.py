@@ -2,6 +2,10 @@
 and on one that every form a wrapper accepts -- strides, given outputs, row-major and packed operands,
 int32 and bf16 results, stored and missing workspaces -- gives bit for bit what the wrapper's own code
 gives, and that what the wrapper refuses stays refused with the same error."""
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -53,6 +57,16 @@ def test_a_launch_that_fails_is_raised_and_not_run_again(monkeypatch):
                 lambda: npu_kernels.mm_i8(t, w, t)):
         with pytest.raises(_lib.W8A8Error, match="EHIP"):
             run()
+
+
+def test_an_exception_inside_the_call_leaves_the_interpreter_whole():
+    """A C++ exception while the GIL is released (a tensor without storage, ..) declines, with the GIL held
+    again.  In a process of its own: without it the interpreter aborts."""
+    code = ("import torch\nfrom w8a8 import _lib\nn = _lib.launch_module()\n"
+            "assert [n.settle('w8a8_k_in', -1) for _ in range(100)] == [None] * 100\nprint('whole')")
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100,
+                       env={**os.environ, "PYTHONPATH": os.path.dirname(os.path.dirname(ops.__file__))})
+    assert r.returncode == 0 and "whole" in r.stdout, r.stderr
 
 
 def both(monkeypatch, call):
@@ -158,3 +172,17 @@ def test_refusals_are_the_wrappers(monkeypatch):
             return e.type, str(e.value)
         a, b = both(monkeypatch, refused)
         assert a == b, i
+
+
+@pytest.mark.gpu
+def test_transformed_tensors_are_refused_as_by_the_wrappers(monkeypatch):
+    """torch.func wraps tensors without a storage of their own: the error is the one of the wrapper's code."""
+    gw, sw = ops.pack_gemv_weight(torch.ones(96, 128, dtype=torch.int8, device=DEV)), torch.ones(96, device=DEV)
+    x = bf(3, 1, 128)
+
+    def refused():
+        with pytest.raises(RuntimeError) as e:
+            torch.func.vmap(lambda r: ops.gemv_bf16(r, gw, sw))(x)
+        return e.type, str(e.value)
+    a, b = both(monkeypatch, refused)
+    assert a == b
