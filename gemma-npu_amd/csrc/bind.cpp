@@ -192,7 +192,11 @@ PyObject* linear(PyObject* const* a) {
     need(a[7] == Py_None);
   }
   const uint16_t* rw = nullptr;
-  if (a[8] != Py_None) rw = bf(c.vec(a[8], at::kBFloat16));
+  if (a[8] != Py_None) {
+    const Tensor& r = c.vec(a[8], at::kBFloat16);
+    need(epi != 3 || r.size(0) >= N);
+    rw = bf(r);
+  }
   const float eps = real(a[9]);
   const Tensor y = output(c, a[10], M, epi == 1 ? I : N, at::kBFloat16);
   // the C entry checks a given workspace's size

@@ -555,6 +555,8 @@ def linear_bf16(x, w, sw=None, epilogue="none", residual=None, rms_w=None, eps=1
     rwp = None
     if rms_w is not None:
         _check(rms_w, "rms_w", torch.bfloat16, 1)
+        if epi == 3 and rms_w.shape[0] < w.N:
+            raise ValueError(f"linear_bf16: rms_w has {rms_w.shape[0]} values for {w.N} columns")
         rwp = rms_w.data_ptr()
     need = linear_workspace_bytes(M, w.N, K)
     ws = workspace(x.device, need) if ws_arg is None else ws_arg
@@ -616,6 +618,8 @@ def gemv_bf16(x, w, s, out=None):
     if out is None:
         out = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
     _check(out, "out", torch.bfloat16)
+    if out.shape[0] < M or out.shape[1] < N:
+        raise ValueError(f"gemv_bf16: out has shape {tuple(out.shape)}, the result {(M, N)}")
     wt = w.data if packed else w
     _same_device(x, wt, s, out)
     if packed:

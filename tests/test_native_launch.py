@@ -150,6 +150,27 @@ def test_equals_the_wrappers_own_code(monkeypatch):
                 assert torch.equal(a.float().nan_to_num(), b.float().nan_to_num()), name
 
 
+def short_operands(x, pw, gw, w, sw, res, rms_w):
+    """Calls with a norm weight shorter than the row, or an output smaller than the result."""
+    return [lambda: ops.linear_bf16(x, pw, epilogue="residual_rms", residual=res, rms_w=rms_w),
+            lambda: ops.gemv_bf16(x, gw, sw, res[:1]), lambda: ops.gemv_bf16(x, gw, sw, res[:, :95]),
+            lambda: ops.gemv_bf16(x, w, sw, res.view(1, -1))]
+
+
+def test_short_operands_are_refused_before_the_call(monkeypatch):
+    def call(*a):
+        raise AssertionError("launched")
+    monkeypatch.setattr(ops, "_native", None)
+    monkeypatch.setattr(ops, "_check", lambda *a: None)  # the device
+    monkeypatch.setattr(ops, "call", call)
+    x, res = torch.zeros(2, 128, dtype=torch.bfloat16), torch.zeros(2, 96, dtype=torch.bfloat16)
+    w, sw = torch.zeros(96, 128, dtype=torch.int8), torch.zeros(96)
+    pw, gw = ops.PackedWeight(w, 96, 128, sw=sw), ops.GemvWeight(w, 96, 128)
+    for run in short_operands(x, pw, gw, w, sw, res, res[0, :95]):
+        with pytest.raises(ValueError):
+            run()
+
+
 @pytest.mark.gpu
 def test_refusals_are_the_wrappers(monkeypatch):
     w = torch.ones(96, 128, dtype=torch.int8, device=DEV)
@@ -157,7 +178,7 @@ def test_refusals_are_the_wrappers(monkeypatch):
     pw, gw, x = ops.pack_weight(w, "nk", sw=sw), ops.pack_gemv_weight(w), bf(2, 128)
     h = bf(4, 40, 128)
     small = torch.empty(8, dtype=torch.uint8, device=DEV)
-    calls = [lambda: ops.gemv_bf16(x.float(), gw, sw), lambda: ops.gemv_bf16(x[:, :64], gw, sw),
+    calls = [*short_operands(x, pw, gw, w, sw, bf(2, 96), bf(95)), lambda: ops.gemv_bf16(x.float(), gw, sw), lambda: ops.gemv_bf16(x[:, :64], gw, sw),
              lambda: ops.linear_bf16(x, pw, ws_arg=small),
              lambda: ops.gemv_bf16(bf(17, 128), gw, sw), lambda: ops.gemv_bf16(x.cpu(), gw, sw),
              lambda: ops.linear_bf16(bf(128, 2).t(), pw), lambda: ops.linear_bf16(x, pw, epilogue="residual"),
