@@ -1,5 +1,5 @@
-"""Builds libw8a8.so (every HIP source under csrc/) for gfx950 with hipcc, and _launch.so (the
-wrappers' launch path, csrc/bind.cpp) with g++.
+"""Builds libw8a8.so (every HIP source under csrc/) for gfx950 with hipcc, and, where g++ and a ROCm torch
+with its headers are there, the _launch module (the wrappers' launch path, csrc/bind.cpp).
 
 Run as `python -m w8a8.build` from gemma-npu_amd/, or through __graft_entry__.build().
 Objects go to gemma-npu_amd/_build/, the library next to this file.
@@ -7,8 +7,10 @@ Objects go to gemma-npu_amd/_build/, the library next to this file.
 import concurrent.futures
 import glob
 import os
+import shutil
 import subprocess
 import sys
+import sysconfig
 
 PKG = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(PKG)
@@ -16,7 +18,7 @@ CSRC = os.path.join(ROOT, "csrc")
 INCLUDE = os.path.join(os.path.dirname(ROOT), "include")
 BUILD = os.path.join(ROOT, "_build")
 LIB = os.path.join(PKG, "libw8a8.so")
-LAUNCH = os.path.join(PKG, "_launch.so")
+LAUNCH = os.path.join(PKG, "_launch" + sysconfig.get_config_var("EXT_SUFFIX"))
 ARCH = "gfx950"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -41,11 +43,17 @@ def _compile(src):
 
 
 def _build_launch():
-    """csrc/bind.cpp (host code against torch's headers) -> w8a8/_launch.so, linked to libw8a8.so."""
-    import sysconfig
-
-    import torch
-    from torch.utils import cpp_extension
+    """csrc/bind.cpp (host code against torch's headers) -> LAUNCH, linked to libw8a8.so.  Returns None, or why
+    it was left out: the wrappers then make every call through ctypes."""
+    try:
+        import torch
+        from torch.utils import cpp_extension
+    except ImportError as e:
+        return f"{e}"
+    if not torch.version.hip:
+        return "torch is not built for ROCm"
+    if not shutil.which("g++"):
+        return "no g++"
     rocm = os.path.dirname(os.path.dirname(HIPCC))
     include = [*cpp_extension.include_paths(), os.path.join(rocm, "include"), sysconfig.get_paths()["include"], INCLUDE]
     tmp = LAUNCH + ".tmp"
@@ -56,8 +64,9 @@ def _build_launch():
            "-Wl,-rpath,$ORIGIN"]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
-        raise RuntimeError(f"g++ failed on bind.cpp:\n{r.stdout}\n{r.stderr}")
+        return f"g++ failed on bind.cpp:\n{r.stdout}\n{r.stderr}"
     os.replace(tmp, LAUNCH)
+    return None
 
 
 def build(verbose=False):
@@ -70,10 +79,15 @@ def build(verbose=False):
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{r.stdout}\n{r.stderr}")
+    # no launch path of another build beside the new library, whatever becomes of this one's
+    for old in glob.glob(os.path.join(PKG, "_launch*.so")):
+        os.remove(old)
     os.replace(tmp, LIB)
-    _build_launch()
+    left_out = _build_launch()
+    if left_out:
+        print(f"{LAUNCH} left out, the wrappers call through ctypes: {left_out}", flush=True)
     if verbose:
-        print(f"built {LIB} from {len(srcs)} sources and {LAUNCH}", flush=True)
+        print(f"built {LIB} from {len(srcs)} sources" + ("" if left_out else f" and {LAUNCH}"), flush=True)
     return LIB
 
 

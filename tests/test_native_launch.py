@@ -10,7 +10,7 @@ import pytest
 import torch
 
 import npu_kernels
-from w8a8 import _lib, attention, fused, ops
+from w8a8 import _lib, attention, build, fused, ops
 
 DEV = "cuda"
 
@@ -26,6 +26,16 @@ def test_declines_what_it_does_not_take():
     assert n.quant_packed(torch.nn.Parameter(x)) is None
     assert n.attention(x, x, x, 0, 0, 1.0, {}) is None
     assert n.wait_stream(x) is None
+
+
+def test_the_build_without_its_tools_leaves_it_out(monkeypatch, tmp_path):
+    monkeypatch.setattr(build, "LAUNCH", str(tmp_path / "_launch.so"))
+    with monkeypatch.context() as m:
+        m.setattr(build.shutil, "which", lambda name: None)
+        assert "g++" in build._build_launch()
+    monkeypatch.setattr(torch.version, "hip", None)
+    assert "ROCm" in build._build_launch()
+    assert not list(tmp_path.iterdir())
 
 
 def test_a_launch_that_fails_is_raised_and_not_run_again(monkeypatch):
