@@ -579,4 +579,13 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_launch", "The wrappers' launch pa
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__launch() { return PyModule_Create(&module); }
+// What the module fits, compared by _lib.launch_module before anything here is called.
+PyMODINIT_FUNC PyInit__launch() {
+  PyObject* m = PyModule_Create(&module);
+  if (m && (PyModule_AddStringConstant(m, "torch_build", W8A8_TORCH) < 0 ||
+            PyModule_AddStringConstant(m, "sources", W8A8_SOURCES) < 0)) {
+    Py_DECREF(m);
+    return nullptr;
+  }
+  return m;
+}

@@ -5,6 +5,7 @@ ctypes releases the GIL for the duration of each foreign call, so launches from 
 thread overlap with Python work on other threads.
 """
 import ctypes
+import hashlib
 import os
 import threading
 
@@ -131,14 +132,36 @@ def lib():
     return _lib
 
 
+def torch_build():
+    """The torch build whose tensor layout and symbols the launch path is compiled against."""
+    import torch
+    return f"{torch.__version__} {torch.version.git_version}"
+
+
+def launch_sources():
+    """Digest of what the launch path is compiled from, or None where the sources are not shipped."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    h = hashlib.sha256()
+    try:
+        for path in (os.path.join(os.path.dirname(root), "include", "w8a8.h"), os.path.join(root, "csrc", "bind.cpp")):
+            with open(path, "rb") as f:
+                h.update(f.read())
+    except OSError:
+        return None
+    return h.hexdigest()
+
+
 def launch_module():
-    """The native launch path (csrc/bind.cpp, w8a8/_launch.so), or None if it is not built or does not
-    fit this torch: the wrappers then make every call through ctypes, with the same results."""
+    """The native launch path (csrc/bind.cpp, the _launch module), or None if it is not built, or was built
+    for another CPython (its file name), another torch or from other sources than those here: the wrappers
+    then make every call through ctypes, with the same results."""
     try:
         from . import _launch
     except ImportError:
         return None
-    return _launch
+    if getattr(_launch, "torch_build", None) != torch_build():
+        return None
+    return _launch if launch_sources() in (None, getattr(_launch, "sources", None)) else None
 
 
 def call(name, *args):

@@ -48,6 +48,8 @@ def _build_launch():
     try:
         import torch
         from torch.utils import cpp_extension
+
+        from w8a8 import _lib
     except ImportError as e:
         return f"{e}"
     if not torch.version.hip:
@@ -57,7 +59,9 @@ def _build_launch():
     rocm = os.path.dirname(os.path.dirname(HIPCC))
     include = [*cpp_extension.include_paths(), os.path.join(rocm, "include"), sysconfig.get_paths()["include"], INCLUDE]
     tmp = LAUNCH + ".tmp"
+    fits = {"W8A8_TORCH": _lib.torch_build(), "W8A8_SOURCES": _lib.launch_sources()}
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+           *(f'-D{k}="{v}"' for k, v in fits.items()),
            *(f"-isystem{d}" for d in include), os.path.join(CSRC, "bind.cpp"), "-o", tmp,
            f"-L{os.path.join(os.path.dirname(torch.__file__), 'lib')}", "-ltorch_python", "-ltorch", "-ltorch_cpu",
            "-ltorch_hip", "-lc10", "-lc10_hip", f"-L{os.path.join(rocm, 'lib')}", "-lamdhip64", f"-L{PKG}", "-lw8a8",
@@ -92,5 +96,6 @@ def build(verbose=False):
 
 
 if __name__ == "__main__":
+    sys.path.insert(0, ROOT)
     build(verbose=True)
     sys.exit(0)

@@ -28,6 +28,19 @@ def test_declines_what_it_does_not_take():
     assert n.wait_stream(x) is None
 
 
+def test_a_module_that_does_not_fit_is_not_used(monkeypatch):
+    n = _lib.launch_module()
+    for name in ("torch_build", "sources"):
+        with monkeypatch.context() as m:
+            m.setattr(n, name, "another")
+            assert _lib.launch_module() is None
+        with monkeypatch.context() as m:
+            m.delattr(n, name)
+            assert _lib.launch_module() is None
+    monkeypatch.setattr(_lib, "launch_sources", lambda: None)  # not shipped: nothing to compare
+    assert _lib.launch_module() is n
+
+
 def test_the_build_without_its_tools_leaves_it_out(monkeypatch, tmp_path):
     monkeypatch.setattr(build, "LAUNCH", str(tmp_path / "_launch.so"))
     with monkeypatch.context() as m:
