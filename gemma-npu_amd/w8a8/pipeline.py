@@ -396,13 +396,15 @@ class Decoder:
             raise ValueError("Decoder: the final norm's eps differs from the layers' rms_norm_eps")
         self.tail_ws = torch.empty(int(lib().w8a8_decode_tail_workspace_bytes(self.cfg.vocab_size)),
                                    dtype=torch.uint8, device=dev)
-        # layers whose few key chunks (a sliding window) the o projection merges in its prologue: rows
-        # up to 2048, where one launch beats two (8 heads of 256, 8 chunks: attention, merge and o
-        # 12.0 us against 12.5); at 8 heads of 512 every workgroup reads twice the partials (16 chunks:
-        # 18.7 us against 14.4 with the merge kernel)
+        # layers whose key chunks' partials the o projection merges in its prologue.  Every workgroup then
+        # reads them all, heads * head_dim * chunks values: attention, merge and o of 8 heads of 256 at
+        # hidden 1536, us fused / with the merge kernel: 1 chunk 10.6 / 11.7, 4 chunks (8192) 10.9 / 11.6,
+        # 8 chunks 11.6 / 11.6, 16 chunks 12.9 / 11.8; hidden 2560 11.8 / 12.0 at 8192, 12.7 / 12.0 at
+        # 16384; 8 heads of 512 never faster (2 chunks, 8192: 13.8 / 13.6)
         self.merge_in_o = {p.index for p in prefill.plans
                            if p.heads // p.kv_heads <= 8 and p.heads * p.head_dim <= 2048
-                           and attention.decode_grid_chunks(p.head_dim, self.max_len, p.window) <= 16}
+                           and p.heads * p.head_dim
+                           * attention.decode_grid_chunks(p.head_dim, self.max_len, p.window) <= 8192}
         # the residual stream's norms as the prologue of the linear that reads them (hidden <= 1536)
         self.fuse_norms = self.cfg.hidden_size <= 1536 and self.cfg.hidden_size % 16 == 0
         self.length = None

@@ -107,6 +107,22 @@ def test_norm_prologues_match_the_row_kernels():
 
 
 @torch.inference_mode()
+def test_merge_in_the_o_projection_follows_the_cache_length():
+    """A cache of few key chunks merges them in the o projection, a longer one of the full layers with the
+    merge kernel: the same logits bit for bit."""
+    from w8a8.pipeline import Decoder, Prefill
+    ours = engine_model(build(seed=43))
+    ids = torch.randint(0, 512, (1, 70), generator=torch.Generator().manual_seed(44))
+    short, long = Decoder(Prefill(ours), max_len=128), Decoder(Prefill(ours), max_len=1024)
+    full = {p.index for p in short.pre.plans if not p.window}
+    assert len(short.merge_in_o) == 10 and long.merge_in_o == short.merge_in_o - full and full
+    short.start(ids)
+    long.start(ids)
+    for i in range(6):
+        assert torch.equal(short.step(), long.step()), f"step {i}"
+
+
+@torch.inference_mode()
 def test_run_like_the_reference():
     """pipeline.run with gemma_npu.py:271-296's signature and results: (ttft, decode tok/s, tokens,
     last-token logits).  With the engine's Prefill its tokens are a Decoder's (the first the argmax of
