@@ -1,7 +1,8 @@
 """The native launch path of the torch-facing wrappers (csrc/bind.cpp): what it declines without a GPU,
 and on one that every form a wrapper accepts -- strides, given outputs, row-major and packed operands,
-int32 and bf16 results, stored and missing workspaces -- gives bit for bit what the wrapper's own code
-gives, and that what the wrapper refuses stays refused with the same error."""
+int32 and bf16 results, stored and missing workspaces -- is taken or declined as stated and gives bit for
+bit what the wrapper's own code gives, and that what the wrapper refuses stays refused with the same error.
+"""
 import os
 import subprocess
 import sys
@@ -92,10 +93,24 @@ def test_an_exception_inside_the_call_leaves_the_interpreter_whole():
     assert r.returncode == 0 and "whole" in r.stdout, r.stderr
 
 
-def both(monkeypatch, call):
+class Recorded:
+    """The native module; `taken` holds for each call made through it whether it was taken."""
+
+    def __init__(self, module):
+        self.module, self.taken = module, []
+
+    def __getattr__(self, name):
+        def run(*a):
+            r = getattr(self.module, name)(*a)
+            self.taken.append(r is not None)
+            return r
+        return run
+
+
+def both(monkeypatch, call, native=None):
     """call() on the native path and on the wrappers' own code."""
     outs = []
-    for native in (_lib.launch_module(), None):
+    for native in (native or _lib.launch_module(), None):
         for m in (ops, fused, attention):
             monkeypatch.setattr(m, "_native", native)
         outs.append(call())
@@ -130,6 +145,11 @@ def forms():
     cs, yq = bf(33, 128, seed=6), bf(33, 4 * 128, seed=7)
     qa, k, v = bf(2, 40, 128, seed=8), bf(1, 40, 128, seed=9), bf(1, 40, 128, seed=10)
     qt = bf(40, 2, 128, seed=11).transpose(0, 1)  # [H, T, D] with rows H * D apart
+    # causal calls whose key ranges are split: their parts need a workspace
+    qs, ks, vs = bf(8, 512, 256, seed=12), bf(1, 512, 256, seed=13), bf(1, 512, 256, seed=14)
+    ql, kl, vl = bf(8, 2048, 256, seed=15), bf(1, 2048, 256, seed=16), bf(1, 2048, 256, seed=17)
+    for T in (512, 2048):
+        assert _lib.lib().w8a8_attention_workspace_bytes(8, 1, T, T, 256, 0, 0) > 0
     return {
         "gemv": lambda: ops.gemv_bf16(one, gw, sw), "gemv bf16 scales": lambda: ops.gemv_bf16(one, gw, sw.bfloat16()),
         "gemv strided out": lambda: ops.gemv_bf16(x[:3], gw, sw, torch.zeros(3, 128, dtype=torch.bfloat16, device=DEV)[:, :96]),
@@ -154,23 +174,40 @@ def forms():
         "k_qkv shared": lambda: fused.k_qkv(yq, None, None, cs, cs, None, None, 1e-6, 4, 0, 128, True),
         "attention": lambda: attention.attention(qa, k, v), "attention window": lambda: attention.attention(qa, k, v, 0, 16),
         "attention strided": lambda: attention.attention(qt, k, v, 0, 0, 0.5),
+        "attention split": lambda: attention.attention(qs, ks, vs),
         "attention_quant": lambda: attention.attention_quant(qa, k, v),
+        "attention_quant two steps": lambda: attention.attention_quant(qs, ks, vs),
+        "attention_quant split": lambda: attention.attention_quant(ql, kl, vl),
         "decode": lambda: attention.decode(qa[:, -1], k, v, None, 8), "decode 3-D": lambda: attention.decode(qa[:, -1:], k, v),
     }
+
+
+# What the native path leaves to the wrapper: all of a form's native calls, or, where the stream has no
+# workspace stored yet, the first one alone.
+DECLINED = {"linear unused residual", "k_ple_out number", "decode 3-D"}
+NO_WORKSPACE_YET = {"attention split", "attention_quant split", "decode"}
 
 
 @pytest.mark.gpu
 def test_equals_the_wrappers_own_code(monkeypatch):
     for name, call in forms().items():
         print(f"native launch path: {name}", flush=True)
-        got, want = (flat(r) for r in both(monkeypatch, call))
-        assert len(got) == len(want), name
-        for a, b in zip(got, want):
-            assert a.shape == b.shape and a.dtype == b.dtype and a.stride() == b.stride(), name
-            if a.dtype == torch.int8 and a.dim() == 1:  # packed rows: the padding of the last block is zero in both
-                assert torch.equal(a, b), name
+        monkeypatch.setattr(attention, "_WS", {})
+        monkeypatch.setattr(attention, "_SPLIT_WS", {})
+        for again in (False, True):
+            native = Recorded(_lib.launch_module())
+            got, want = (flat(r) for r in both(monkeypatch, call, native))
+            if name == "attention_quant two steps":  # the fused call declined, attention and then no k_attn_out
+                assert native.taken == [False, again]
             else:
-                assert torch.equal(a.float().nan_to_num(), b.float().nan_to_num()), name
+                assert native.taken == [name not in DECLINED and (again or name not in NO_WORKSPACE_YET)], name
+            assert len(got) == len(want), name
+            for a, b in zip(got, want):
+                assert a.shape == b.shape and a.dtype == b.dtype and a.stride() == b.stride(), name
+                if a.dtype == torch.int8 and a.dim() == 1:  # packed rows: the padding of the last block is zero in both
+                    assert torch.equal(a, b), name
+                else:
+                    assert torch.equal(a.float().nan_to_num(), b.float().nan_to_num()), name
 
 
 def short_operands(x, pw, gw, w, sw, res, rms_w):
@@ -201,7 +238,8 @@ def test_refusals_are_the_wrappers(monkeypatch):
     pw, gw, x = ops.pack_weight(w, "nk", sw=sw), ops.pack_gemv_weight(w), bf(2, 128)
     h = bf(4, 40, 128)
     small = torch.empty(8, dtype=torch.uint8, device=DEV)
-    calls = [*short_operands(x, pw, gw, w, sw, bf(2, 96), bf(95)), lambda: ops.gemv_bf16(x.float(), gw, sw), lambda: ops.gemv_bf16(x[:, :64], gw, sw),
+    calls = [*short_operands(x, pw, gw, w, sw, bf(2, 96), bf(95)),
+             lambda: ops.gemv_bf16(x.float(), gw, sw), lambda: ops.gemv_bf16(x[:, :64], gw, sw),
              lambda: ops.linear_bf16(x, pw, ws_arg=small),
              lambda: ops.gemv_bf16(bf(17, 128), gw, sw), lambda: ops.gemv_bf16(x.cpu(), gw, sw),
              lambda: ops.linear_bf16(bf(128, 2).t(), pw), lambda: ops.linear_bf16(x, pw, epilogue="residual"),
