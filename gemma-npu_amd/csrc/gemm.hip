@@ -1261,12 +1261,14 @@ static bool pipe_tail_is_short(int M, int NP) {
 //    weight half as often, unless its last round would be nearly empty.
 //
 // This rule is taken below 512 rows, and from K = 2048 on for every row count.  For short-K GEMMs of 512
-// rows and more the configuration of a shape is a stated result of w8a8_gemm_pick_tile_config, and stays:
+// rows and more the choice that was measured before it stays, shape by shape as tests/test_abi.py holds it:
 // up to 1024 rows small tiles by N (64x256 with GELU: gate/up at M = 512 16.2); past that one round of the
 // smallest BMx256 tile where the busiest CU moves fewer bytes than on 64x128, three per CU, else 6, or
-// 64x128 (0) where 6's tiles are fewer than the CUs or leave a nearly empty last round.  The one-round
-// rule would be faster for some of them (1536 x 5120 at M = 1100: 14.1 against 17.4; 1536 x 256 at
-// M = 3658: 6.4 against 8.7).
+// 64x128 (0) where 6's tiles are fewer than the CUs or leave a nearly empty last round.  So the line at 512
+// rows is where those measurements begin, not where the hardware changes: of the shapes behind it some
+// would be faster on another tile (K = 1536: N = 2048 at M = 512 8.4, 6.6 on 64x64 with four waves; 6144 at
+// 768 15.6, 12.1 on 96x256; gate/up with GELU at 768 22.9, 21.0 on 160x256; 5120 at 1100 17.4, 13.4 on 96x256;
+// 256 at 3658 9.0, 6.5 on 64x64 with four waves).
 int gemm_pick_config(int M, int NP, int K, int epi) {
   const int cus = cu_count();
   auto tiles = [&](int bm, int bn) { return int64_t((M + bm - 1) / bm) * ((NP + bn - 1) / bn); };
