@@ -526,8 +526,9 @@ __global__ __launch_bounds__(PRO == 4 ? 1024 : 768) void gemv1_kernel(GemvParams
   if (threadIdx.x < 2) *reinterpret_cast<v4i*>(xs + XS + 8 * threadIdx.x) = v4i{0, 0, 0, 0};
   v4i wv[U][TPW];
   if constexpr (PRO == 5) {
-    // The row's pieces of 8 are asked for before the weights, two per thread (all of it from 12 waves
-    // on); a wait inside a loop would be one for the weights too.
+    // The row's pieces of 8 are asked for before the weights, two per thread: a row of up to 8192 elements
+    // at eight waves, 4096 at four.  What a longer one has past that is copied first, in a loop that waits for
+    // each piece before any weight is asked for.
     const int k0 = int(threadIdx.x) * 8, nt8 = int(blockDim.x) * 8, k1 = k0 + nt8;
     for (int k = k1 + nt8; k < row_end; k += nt8)
       *reinterpret_cast<v4i*>(xs + k) = buf_load16(rx, k < p.K ? uint32_t(k) * 2u : PAST);
