@@ -687,7 +687,9 @@ static void gemv_launch_few(const GemvParams& p, int64_t groups, hipStream_t str
 // unit cost the gate/up GEMV 1-2 us more), and more waves only cost barriers (down 6144 x 1536 in halves:
 // 16 waves 5.5 us, 8 waves 4.7, 6 waves 5.5).  The partial sums depend on (N, K) alone; the units per
 // workgroup, which change no sum, are one, or with a row to make (the norm, the merge) up to twelve waves'
-// worth, so that the row is made less often (gate/up 1536 x 12288: 8.4 us with one, 7.5 with three).
+// worth, so that the row is made less often (gate/up 1536 x 12288: 8.4 us with one, 7.5 with three), eight
+// waves' from 2048 tiles on, where a CU has several such workgroups anyway (33000 x 256 with its norm 6.1 ->
+// 5.9 us, 65504 x 128 7.7 -> 7.35; 20000 x 128 with GELU 4.8 with twelve, 5.3 with eight).
 // Sets units, split and gpb; the kernel's R, or 0 for HALF.
 static int gemv1_plan(GemvParams& p, bool make_row) {
   const int cus = gemv_cu_count();
@@ -697,7 +699,7 @@ static int gemv1_plan(GemvParams& p, bool make_row) {
   const int parts = few_tile_split(ntiles, p.KB);  // a power of two, above 8 only at one unit per CU
   p.units = half ? (p.N + 7) / 8 : ntiles;
   p.split = half ? max(parts / 2, 1) : min(per_cu == 1 ? 8 : 4, parts);
-  p.gpb = make_row ? min(per_cu, 12 / p.split) : 1;
+  p.gpb = make_row ? min(per_cu, (per_cu < 8 ? 12 : 8) / p.split) : 1;
   return half ? 0 : parts / p.split;
 }
 
@@ -712,7 +714,8 @@ static bool gemv1_takes(const GemvParams& p) {
 // U fragments in flight per wave: all of a wave's share in one round where the registers allow it (seven or
 // eight steps in one round of 8 rather than 12: 4096 x 4096 6.4 -> 6.1 us, row-major 7.4 -> 7.0, N = 16384,
 // K = 2048 9.6 -> 8.5).  With the norm six at most, whose 80 registers let two workgroups of twelve waves
-// stand on a CU (N = 32768, K = 1536, two waves per unit: 18.2 us in rounds of 12, 14.2 in rounds of 6).
+// stand on a CU, and four from 2048 tiles on (one or two waves per unit: N x K 32768 x 1536 18.2 us in rounds
+// of 12 fragments, 14.2 in rounds of 6, 11.6 in rounds of 4 with eight waves; 40000 x 1024 11.8 -> 11.1).
 // MI355X, weights cold, a chain of launches replayed from a graph (a chain of empty ones takes 1.9 us
 // each), us per launch, before (one tile per workgroup of 8 or 16 waves, the row made by one wave, the
 // scales fetched after the sums) -> now: o 2048 x 1536 4.5 -> 3.3, 4096 x 1536 5.5 -> 4.0; qkv 1536 x
@@ -749,7 +752,7 @@ static void gemv1_launch(const GemvParams& p0, hipStream_t stream) {
   if (per_wave <= 1) W8A8_GEMV1(1);
   else if (per_wave <= 2) W8A8_GEMV1(2);
   else if (per_wave <= 3) W8A8_GEMV1(3);
-  else if (per_wave <= 4 || (ACT == 1 && half)) W8A8_GEMV1(4);
+  else if (per_wave <= 4 || (ACT == 1 && half) || (PRO <= 3 && p.split < 4)) W8A8_GEMV1(4);
   else if (per_wave <= 6 || half || PRO != 5) W8A8_GEMV1(6);
   else if (per_wave <= 8) W8A8_GEMV1_WHOLE(8);
   else W8A8_GEMV1_WHOLE(PRO != 5 ? 8 : 12);

@@ -394,3 +394,23 @@ def test_gemv_a_row_has_the_same_bits_alone_and_among_others(N, K):
                  lambda r: ops.gemv_act_bf16(x[:r], pw, s, "gelu_mul", mul=mul[:r]),
                  *([lambda r: ops.gemv_act_bf16(x[:r], pw, s, "gelu_pair")] if N % 32 == 0 else [])):
         assert torch.equal(call(1), call(5)[:1])
+
+
+@pytest.mark.parametrize("I, K", [(16384, 1536), (20000, 1040), (32752, 128), (16384, 64)])
+def test_gemv_norm_of_wide_weights(I, K):
+    """From 2048 tiles on a unit has one or two waves: the norm prologue, plain and with the GELU pair, against
+    the row kernel followed by the GEMV, bit for bit."""
+    g = torch.Generator(device=DEV).manual_seed(I + K)
+    w = torch.randint(-127, 128, (2 * I, K), generator=g, dtype=torch.int8, device=DEV)
+    pw = ops.pack_gemv_weight(w)
+    s = torch.rand(2 * I, generator=g, device=DEV) * 0.01
+    y, r = (torch.randn(1, K, generator=g, device=DEV).to(torch.bfloat16) for _ in range(2))
+    w1, w2 = ((1 + 0.1 * torch.randn(K, generator=g, device=DEV)).to(torch.bfloat16) for _ in range(2))
+    print(f"wide norm GEMV I={I} K={K}", flush=True)
+    h, x = ops.rms_residual_norm(y, r, w1, w2, 1e-6)
+    want = ops.gemv_bf16(x, pw, s)
+    got, gh = ops.gemv_norm_bf16(y, r, w1, 1e-6, pw, s, w2=w2)
+    assert torch.equal(gh, h) and torch.equal(got, want)
+    got, _ = ops.gemv_norm_bf16(y, r, w1, 1e-6, pw, s, act="gelu_pair", w2=w2)
+    gate, up = want.view(2, I // 16, 16)
+    assert torch.equal(got.view(-1, 16), ops.gelu_mul_bf16(gate, up))
